@@ -1,7 +1,7 @@
-// The C_l emulator's network (include/crime_mlp.h): BF16 MFMA forward/backward GEMMs with fused
-// epilogues, FP32 edge layers, deterministic split-K weight gradients reduced inside Adam, and one
-// training step captured as a HIP graph (step counter, learning rate and minibatch RNG live on the
-// device, so the graph replays unchanged).
+// The C_l emulator's network (include/crime_mlp.h): one kernel takes a block of rows through every layer
+// (BF16 MFMA, FP32 edge layers, activations in LDS), and in training back through them; a second one forms the
+// deterministic split-K weight gradients and applies Adam.  A training step is those two, captured as a HIP
+// graph (step counter, learning rate and minibatch RNG live on the device, so the graph replays unchanged).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdarg.h>
@@ -9,6 +9,7 @@
 #include <string.h>
 
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "crime_mlp.h"
@@ -34,11 +35,13 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 // per-handle device state read by the captured step
 struct DevState {
   int step;        // Adam updates applied since set_params
+  int step_b;      // k_mlp_rows' copy of step for k_mlp_update, which advances step itself
   int local;       // step index within the current train call (loss slot)
   int total;       // steps of the cosine schedule
   float lr0, b1, b2, eps;
   uint32_t seed;
   int64_t ndata;
+  float lr, c1, c2;   // this step's learning rate and Adam bias corrections (k_mlp_rows, for k_mlp_update)
 };
 
 __device__ __forceinline__ uint16_t f2bf(float x)
@@ -49,260 +52,491 @@ __device__ __forceinline__ uint16_t f2bf(float x)
   return (uint16_t)(u >> 16);
 }
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
-__device__ __forceinline__ float sigm(float z) { return 1.0f / (1.0f + expf(-z)); }
 
-// ---------------------------------------------------------------------------------------------
-// BF16 GEMM C[M x N] = A[M x K] B[K x N] with FP32 accumulation; TA: A is stored K x M, TB: B is
-// stored N x K.  64 x 64 output tile per workgroup (4 waves of 2 x 2 v_mfma_f32_16x16x32_bf16),
-// K in chunks of 32 through LDS, split-K over blockIdx.z (rows [z kchunk, (z+1) kchunk) of K).
-// MFMA operands: lane = i + 16 (k / 4) holds A[i][k] (element k % 4), lane = j + 16 (k / 4) holds
-// B[k][j]; D[i][j] is element i % 4 of lane j + 16 (i / 4).  N and K are multiples of 64 and 32.
-// ---------------------------------------------------------------------------------------------
-constexpr int TM = 64, TN = 64, TK = 32, LP = TK + 8;
-
-template <bool TA, bool TB, class Epi>
-__global__ __launch_bounds__(256) void k_gemm(const uint16_t *__restrict__ A, int lda, const uint16_t *__restrict__ B,
-                                              int ldb, int M, int K, int kchunk, Epi epi)
+// four floats to BF16, round to nearest even: the bits of f2bf in one v_cvt_pk_bf16_f32 per pair
+__device__ __forceinline__ uint2 pack4_bf16(float a, float b, float c, float d)
 {
-  __shared__ __align__(16) uint16_t As[TM * LP];
-  __shared__ __align__(16) uint16_t Bs[TN * LP];   // Bs[n][k]
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int m0 = blockIdx.x * TM, n0 = blockIdx.y * TN;
-  const int kb = blockIdx.z * kchunk;
-  const int ke = K < kb + kchunk ? K : kb + kchunk;
-  const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32;
-  f4 acc[2][2];
-  for (int i = 0; i < 2; i++)
-    for (int j = 0; j < 2; j++) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
-  for (int k0 = kb; k0 < ke; k0 += TK) {
-    if (!TA) {
-      const int m = tid >> 2, k8 = (tid & 3) * 8;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (m0 + m < M) v = *(const uint4 *)(A + (size_t)(m0 + m) * lda + k0 + k8);
-      *(uint4 *)(As + m * LP + k8) = v;
-    } else {
-      const int k = tid >> 3, m8 = (tid & 7) * 8;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (m0 + m8 < M) v = *(const uint4 *)(A + (size_t)(k0 + k) * lda + m0 + m8);
-      const uint16_t *e = (const uint16_t *)&v;
-      for (int i = 0; i < 8; i++) As[(m8 + i) * LP + k] = e[i];
-    }
-    if (!TB) {
-      const int k = tid >> 3, n8 = (tid & 7) * 8;
-      uint4 v = *(const uint4 *)(B + (size_t)(k0 + k) * ldb + n0 + n8);
-      const uint16_t *e = (const uint16_t *)&v;
-      for (int i = 0; i < 8; i++) Bs[(n8 + i) * LP + k] = e[i];
-    } else {
-      const int n = tid >> 2, k8 = (tid & 3) * 8;
-      *(uint4 *)(Bs + n * LP + k8) = *(const uint4 *)(B + (size_t)(n0 + n) * ldb + k0 + k8);
-    }
-    __syncthreads();
-    // gfx950's v_mfma_f32_16x16x32_bf16: the whole 32-deep k tile in one instruction per 16 x 16 block.
-    // Lane l supplies A[row l % 16][k 8 (l / 16) .. +7] and B[k 8 (l / 16) .. +7][column l % 16].
-    {
-      bf16x8 af[2], bfr[2];
-      for (int i = 0; i < 2; i++)
-        af[i] = __builtin_bit_cast(bf16x8, *(const uint4 *)(As + (wr + 16 * i + (lane & 15)) * LP + 8 * (lane >> 4)));
-      for (int j = 0; j < 2; j++)
-        bfr[j] = __builtin_bit_cast(bf16x8, *(const uint4 *)(Bs + (wc + 16 * j + (lane & 15)) * LP + 8 * (lane >> 4)));
-      for (int i = 0; i < 2; i++)
-        for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-  for (int i = 0; i < 2; i++)
-    for (int j = 0; j < 2; j++)
-      for (int v = 0; v < 4; v++) {
-        const int row = m0 + wr + 16 * i + 4 * (lane >> 4) + v;
-        const int col = n0 + wc + 16 * j + (lane & 15);
-        if (row < M) epi(row, col, acc[i][j][v], (int)blockIdx.z);
-      }
+  typedef float fl4 __attribute__((ext_vector_type(4)));
+  typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+  const fl4 v = {a, b, c, d};
+  return __builtin_bit_cast(uint2, __builtin_convertvector(v, bf4));
 }
 
-// forward: z = acc + b; keep z (FP32) for the backward pass, h = bf16(silu(z))
-struct EpiFwd {
-  const float *bias;
-  float *Z;
-  uint16_t *H;
-  __device__ void operator()(int r, int c, float v, int) const
-  {
-    const float z = v + bias[c];
-    Z[(size_t)r * WD + c] = z;
-    H[(size_t)r * WD + c] = f2bf(z * sigm(z));
-  }
-};
-
-// backward through the layer below: dz_prev = bf16(acc silu'(z_prev)), silu' = s (1 + z (1 - s))
-struct EpiBwd {
-  const float *Zp;
-  uint16_t *dZp;
-  __device__ void operator()(int r, int c, float v, int) const
-  {
-    const float z = Zp[(size_t)r * WD + c], s = sigm(z);
-    dZp[(size_t)r * WD + c] = f2bf(v * s * (1.0f + z * (1.0f - s)));
-  }
-};
-
-// weight gradient: one split's partial sum
-struct EpiPart {
-  float *part;
-  __device__ void operator()(int r, int c, float v, int z) const { part[((size_t)z * WD + r) * WD + c] = v; }
-};
-
-// ---------------------------------------------------------------------------------------------
-// FP32 edge layers, minibatch gather, reductions, Adam
-// ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_in_fwd(const float *__restrict__ X, const float *__restrict__ p, int n,
-                                                float *__restrict__ Z1, uint16_t *__restrict__ H1)
+// 1 / (1 + e^-z) as the correctly rounded quotient: for 1 <= d < 2^120 the reciprocal, one Newton step and two
+// residual corrections give it without the operand scaling of a general division
+__device__ __forceinline__ float sigm(float z)
 {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int r = (int)(idx / WD), c = (int)(idx % WD);
-  if (r >= n) return;
-  float z = p[OFF_W0 + (int64_t)NIN * WD + c];
+  if (__builtin_expect(!(z > -80.0f), 0)) return 1.0f / (1.0f + expf(-z));
+  const float d = 1.0f + expf(-z);
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float r1 = fmaf(fmaf(-d, r, 1.0f), r, r);
+  const float q = fmaf(fmaf(-d, r1, 1.0f), r1, r1);
+  return fmaf(fmaf(-d, q, 1.0f), r1, q);
+}
+
+// bf16(z sigm(z)) of four values.  Most results do not depend on the last bits of sigm: with the hardware's
+// exponential and reciprocal the product is within SILU_ULP units in the last place of z sigm(z) for z > SILU_MIN
+// (checked over every float), so unless it lies that close to a rounding boundary of BF16 its BF16 value is the
+// same.  The others (one in 2600) take sigm.
+constexpr unsigned SILU_ULP = 12;
+constexpr float SILU_MIN = -9.0f;
+__device__ __forceinline__ uint2 silu4_bf16(const float (&z)[4])
+{
+  float h[4];
+  unsigned near = 0xffffu;
+  float low = 0.0f;
 #pragma unroll
-  for (int i = 0; i < NIN; i++) z = fmaf(X[(size_t)r * NIN + i], p[OFF_W0 + (int64_t)i * WD + c], z);
-  Z1[(size_t)r * WD + c] = z;
-  H1[(size_t)r * WD + c] = f2bf(z * sigm(z));
+  for (int v = 0; v < 4; v++) {
+    const float e = __builtin_amdgcn_exp2f(z[v] * -1.44269504088896341f);
+    h[v] = z[v] * __builtin_amdgcn_rcpf(1.0f + e);
+    near = min(near, (__float_as_uint(h[v]) + (SILU_ULP - 0x8000u)) & 0xffffu);
+    low = fminf(low, z[v]);
+  }
+  if (__builtin_expect(near <= 2 * SILU_ULP || !(low > SILU_MIN), 0)) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) h[v] = z[v] * sigm(z[v]);
+  }
+  return pack4_bf16(h[0], h[1], h[2], h[3]);
 }
 
-// one wave per row: y = h5 . w5 + b5; when training also dy = 2 w (y - t) / n, the loss and dz5
-__global__ __launch_bounds__(256) void k_out(const uint16_t *__restrict__ H5, const float *__restrict__ Z5,
-                                             const float *__restrict__ p, const float *__restrict__ T,
-                                             const float *__restrict__ Wt, int n,
-                                             int train, float *__restrict__ Y, float *__restrict__ dy,
-                                             uint16_t *__restrict__ dZ5, const DevState *__restrict__ st,
-                                             float *__restrict__ loss_hist)
+// ---------------------------------------------------------------------------------------------
+// The square layers run on v_mfma_f32_16x16x32_bf16 with the weights as the A operand and the
+// activations as B (D = W^T h^T): lane l supplies W of feature l % 16 at the eight inputs 8 (l / 16) .. + 7,
+// and h of row l % 16 at the same eight; D holds features 4 (l / 16) .. + 3 of row l % 16, four consecutive
+// features of a row, which go back to the LDS tile as one 8-byte store.  The weights' BF16 copies lie in
+// exactly that order, 16 bytes per lane and 1 KB per wave: frag(layer, tile of 16 outputs, step of 32 inputs).
+// wf serves the forward product (outputs n, inputs k), wb the backward one (outputs k, inputs n).
+// ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ size_t frag_index(int layer, int out, int in)
 {
-  const int lane = threadIdx.x & 63;
-  const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= n) return;
-  const float *w5 = p + OFF_W5;
-  float s = 0.f;
-  for (int c = lane; c < WD; c += 64) s = fmaf(bf2f(H5[(size_t)r * WD + c]), w5[c], s);
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  const float y = s + w5[WD];
-  if (!train) {
-    if (lane == 0) Y[r] = y;
+  const int t = out >> 4, s = in >> 5, l = (out & 15) + 16 * ((in & 31) >> 3);
+  return ((((size_t)layer * 16 + t) * 8 + s) * 64 + l) * 8 + (in & 7);
+}
+
+constexpr int UPD_THREADS = 512;
+constexpr int row_threads(int NT) { return 64 * (WD / 16) / NT; }   // a wave per NT tiles of 16 features
+constexpr int HSTR = WD + 8;          // LDS row stride: 16 rows of one 16-byte column fall on distinct banks
+constexpr int TR = RROWS;             // rows per workgroup of a training step: one partial of the column sums
+constexpr int FWD_ROWS = 64;          // rows per workgroup of a large forward call
+static_assert(TR == 32 && WD == 256, "k_mlp_rows' thread layout");
+
+struct RowArgs {
+  const float *X, *T, *Wt;       // inputs, targets, weights (the whole training set with gather)
+  const float *p;
+  const uint16_t *wf, *wb;
+  float *Y;                      // forward only: outputs
+  uint16_t *hp, *dzp;            // training: [4][octet of rows][feature][row % 8]
+  float *part_in, *part_out, *part_b;
+  DevState *st;
+  float *loss;
+  size_t stride;                 // elements per layer of hp, dzp
+  int n, npart;                  // rows; partials allocated per layer in part_b
+  int gather;
+};
+
+// One workgroup takes BM rows through the whole network without leaving the CU: the activations of the
+// current layer stay in one LDS tile, the weights stream from L2 as fragments (prefetched across the
+// epilogue), and a training step (TRAIN) carries on with the loss and the backward pass, its pre-activations
+// held in registers from the forward half.
+// A wave owns NT tiles of 16 features of every row.  What bounds it: up to 32 rows the 128 KB of weights per
+// layer through the CU's vector cache and the latency of the layers in series; at 64 rows the SiLU epilogue
+// (about 12 VALU instructions per element beside 512 MFMA flops), which the second workgroup of the CU overlaps.
+// Measured: 65536 rows forward 82 us (418 TFLOP/s) against 321 us for one kernel per layer, which wrote and
+// read every activation; 128-row workgroups (one per CU) 95 us.  256 rows 13 us (16-row workgroups) against
+// 20 us (32 rows, NT = 2) and 50 us (one kernel per layer).  A training step's rows, 4096 of them: 40 us, and
+// k_mlp_update 13 us, against 480 us for the 30 kernels of a step before.
+template <int BM, int NT, bool TRAIN>
+__global__ __launch_bounds__(row_threads(NT), 4) void k_mlp_rows(RowArgs g)
+{
+  constexpr int MT = BM / 16, NTHREADS = row_threads(NT);
+  constexpr int NZ = TRAIN ? MT : 1;
+  __shared__ __align__(16) uint16_t hs[BM * HSTR];
+  __shared__ __align__(16) float xs[BM * NIN];
+  __shared__ float ds[BM];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lr = lane & 15, lg = lane >> 4;
+  const int row0 = blockIdx.x * BM;
+  const int f0 = 16 * NT * wv + 4 * lg;     // this lane's features: f0 + 16 nt + v
+  uint4 w[NT][8];
+  auto load_w = [&](const uint16_t *frags, int layer) {
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+      for (int s = 0; s < 8; s++)
+        w[nt][s] = *(const uint4 *)(frags + ((((size_t)layer * 16 + NT * wv + nt) * 8 + s) * 64 + lane) * 8);
+  };
+  load_w(g.wf, 0);
+  float tgt = 0.f, wgt = 0.f;          // target and weight of row tid (tid < BM)
+  if (tid < BM) {
+    int64_t i = row0 + tid;
+    const bool live = row0 + tid < g.n;
+    if (TRAIN && g.gather) {
+      u32x4 c = {{(uint32_t)g.st->step, (uint32_t)(row0 + tid), 0u, 0u}};
+      u32x4 r = philox4x32_10(c, g.st->seed, MLP_KEY1);
+      const uint64_t u = ((uint64_t)r.v[0] << 32) | r.v[1];
+      i = (int64_t)(u % (uint64_t)g.st->ndata);
+    }
+    float4 x0 = make_float4(0, 0, 0, 0), x1 = x0;
+    if (live) {
+      x0 = *(const float4 *)(g.X + (size_t)i * NIN);
+      x1 = *(const float4 *)(g.X + (size_t)i * NIN + 4);
+      if (TRAIN) {
+        tgt = g.T[i];
+        wgt = g.Wt[i];
+      }
+    }
+    *(float4 *)(xs + tid * NIN) = x0;
+    *(float4 *)(xs + tid * NIN + 4) = x1;
+  }
+  if (TRAIN && blockIdx.x == 0 && tid == NTHREADS - 1) {
+    const int st = g.st->step, total = g.st->total;
+    const float frac = total > 0 ? fminf((float)st / (float)total, 1.0f) : 0.0f;
+    g.st->step_b = st;
+    g.st->lr = g.st->lr0 * 0.5f * (1.0f + cosf(3.14159265358979f * frac));
+    g.st->c1 = 1.0f - powf(g.st->b1, (float)(st + 1));
+    g.st->c2 = 1.0f - powf(g.st->b2, (float)(st + 1));
+  }
+  __syncthreads();
+
+  float z[NZ][NT][TRAIN ? NH : 1][4];   // pre-activations of every layer (TRAIN)
+  // input layer: z = b + sum_i x_i W0[i], FP32
+#pragma unroll
+  for (int nt = 0; nt < NT; nt++) {
+    const int f = f0 + 16 * nt;
+    float4 wc[NIN];
+#pragma unroll
+    for (int i = 0; i < NIN; i++) wc[i] = *(const float4 *)(g.p + OFF_W0 + (int64_t)i * WD + f);
+    const float4 b = *(const float4 *)(g.p + OFF_W0 + (int64_t)NIN * WD + f);
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      const float4 x0 = *(const float4 *)(xs + (16 * mt + lr) * NIN), x1 = *(const float4 *)(xs + (16 * mt + lr) * NIN + 4);
+      const float x[NIN] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+      float a[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int i = 0; i < NIN; i++) {
+        a[0] = fmaf(x[i], wc[i].x, a[0]);
+        a[1] = fmaf(x[i], wc[i].y, a[1]);
+        a[2] = fmaf(x[i], wc[i].z, a[2]);
+        a[3] = fmaf(x[i], wc[i].w, a[3]);
+      }
+      if constexpr (TRAIN)
+        for (int v = 0; v < 4; v++) z[mt][nt][0][v] = a[v];
+      *(uint2 *)(hs + (16 * mt + lr) * HSTR + f) = silu4_bf16(a);
+    }
+  }
+  __syncthreads();
+
+  // the LDS tile's rows 8 o .. 8 o + 7 of one feature as one 16-byte chunk
+  auto octet = [&](int o, int f) {
+    union { uint16_t e[8]; uint4 q; } u;
+#pragma unroll
+    for (int r = 0; r < 8; r++) u.e[r] = hs[(8 * o + r) * HSTR + f];
+    return u.q;
+  };
+  auto mma = [&](f4 (&acc)[MT][NT]) {
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+      for (int nt = 0; nt < NT; nt++) acc[mt][nt] = (f4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) {
+        const bf16x8 h = __builtin_bit_cast(bf16x8, *(const uint4 *)(hs + (16 * mt + lr) * HSTR + 32 * s + 8 * lg));
+        for (int nt = 0; nt < NT; nt++)
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[nt][s]), h, acc[mt][nt], 0, 0, 0);
+      }
+  };
+
+#pragma unroll
+  for (int k = 0; k < NMID; k++) {
+    if constexpr (TRAIN) {   // the weight gradient's copy of this layer's input
+      const int f = tid & 255;
+#pragma unroll 1
+      for (int o = tid >> 8; o < BM / 8; o += NTHREADS / 256)
+        *(uint4 *)(g.hp + k * g.stride + ((size_t)(row0 / 8 + o) * WD + f) * 8) = octet(o, f);
+    }
+    f4 acc[MT][NT];
+    mma(acc);
+    if (k + 1 < NMID) load_w(g.wf, k + 1);
+    else if (TRAIN) load_w(g.wb, NMID - 1);
+    const float *bias = g.p + OFF_MID + k * MID_STRIDE + (int64_t)WD * WD;
+    __syncthreads();
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+      const int f = f0 + 16 * nt;
+      const float4 b = *(const float4 *)(bias + f);
+      const float bb[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) {
+        float zz[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          zz[v] = acc[mt][nt][v] + bb[v];
+          if constexpr (TRAIN) z[mt][nt][k + 1][v] = zz[v];
+        }
+        *(uint2 *)(hs + (16 * mt + lr) * HSTR + f) = silu4_bf16(zz);
+      }
+    }
+    __syncthreads();
+  }
+
+  // output layer, a wave per row: y = h5 . w5 + b5; training also d = 2 w (y - t) / n and the loss
+  const float *w5 = g.p + OFF_W5;
+  const float o0 = w5[lane], o1 = w5[lane + 64], o2 = w5[lane + 128], o3 = w5[lane + 192], b5 = w5[WD];
+  for (int r = wv; r < BM; r += NTHREADS / 64) {
+    const uint16_t *h = hs + r * HSTR + lane;
+    float s = 0.f;
+    s = fmaf(bf2f(h[0]), o0, s);
+    s = fmaf(bf2f(h[64]), o1, s);
+    s = fmaf(bf2f(h[128]), o2, s);
+    s = fmaf(bf2f(h[192]), o3, s);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == 0) ds[r] = s + b5;
+  }
+  __syncthreads();
+  if constexpr (!TRAIN) {
+    if (tid < BM && row0 + tid < g.n) g.Y[row0 + tid] = ds[tid];
     return;
   }
-  const float e = y - T[r], wt = Wt[r];
-  const float d = 2.0f * wt * e / (float)n;
-  if (lane == 0) {
-    Y[r] = y;
-    dy[r] = d;
-    atomicAdd(loss_hist + st->local, wt * e * e / (float)n);
-  }
-  for (int c = lane; c < WD; c += 64) {
-    const float z = Z5[(size_t)r * WD + c], sg = sigm(z);
-    dZ5[(size_t)r * WD + c] = f2bf(d * w5[c] * sg * (1.0f + z * (1.0f - sg)));
-  }
-}
-
-// partials of dw5 = sum_r h5 dy and db5 = sum_r dy over rows [z RROWS, (z+1) RROWS)
-__global__ __launch_bounds__(256) void k_out_wgrad(const uint16_t *__restrict__ H5, const float *__restrict__ dy, int n,
-                                                   float *__restrict__ part)
-{
-  const int c = threadIdx.x, z = blockIdx.x;
-  const int r0 = z * RROWS, r1 = n < r0 + RROWS ? n : r0 + RROWS;
-  float a = 0.f, b = 0.f;
-  for (int r = r0; r < r1; r++) {
-    const float d = dy[r];
-    a = fmaf(bf2f(H5[(size_t)r * WD + c]), d, a);
-    b += d;
-  }
-  part[(size_t)z * (WD + 1) + c] = a;
-  if (c == 0) part[(size_t)z * (WD + 1) + WD] = b;
-}
-
-// partials of db = sum_r dz (column sums) over one split
-__global__ __launch_bounds__(256) void k_colsum(const uint16_t *__restrict__ dZ, int n, float *__restrict__ part)
-{
-  const int c = threadIdx.x, z = blockIdx.x;
-  const int r0 = z * RROWS, r1 = n < r0 + RROWS ? n : r0 + RROWS;
-  float a = 0.f;
-  for (int r = r0; r < r1; r++) a += bf2f(dZ[(size_t)r * WD + c]);
-  part[(size_t)z * WD + c] = a;
-}
-
-// partials of dW0 = x^T dz1 and db0 = sum_r dz1: part[z][i][c] (i < 8), part[z][8][c]
-__global__ __launch_bounds__(256) void k_in_wgrad(const float *__restrict__ X, const uint16_t *__restrict__ dZ1, int n,
-                                                  float *__restrict__ part)
-{
-  const int c = threadIdx.x, z = blockIdx.x;
-  const int r0 = z * RROWS, r1 = n < r0 + RROWS ? n : r0 + RROWS;
-  float a[NIN + 1] = {};
-  for (int r = r0; r < r1; r++) {
-    const float g = bf2f(dZ1[(size_t)r * WD + c]);
+  else {
+    if (tid < BM) {
+      const float e = ds[tid] - tgt;
+      ds[tid] = 2.0f * wgt * e / (float)g.n;
+      atomicAdd(g.loss + g.st->local, wgt * e * e / (float)g.n);
+    }
+    __syncthreads();
+    // partials of dw5 = sum_r h5 d and db5 = sum_r d over the workgroup's rows
+    if (tid < WD) {
+      float a = 0.f, b = 0.f;
+#pragma unroll 8
+      for (int r = 0; r < BM; r++) {
+        a = fmaf(bf2f(hs[r * HSTR + tid]), ds[r], a);
+        b += ds[r];
+      }
+      g.part_out[(size_t)blockIdx.x * (WD + 1) + tid] = a;
+      if (tid == 0) g.part_out[(size_t)blockIdx.x * (WD + 1) + WD] = b;
+    }
+    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NIN; i++) a[i] = fmaf(X[(size_t)r * NIN + i], g, a[i]);
-    a[NIN] += g;
+    for (int nt = 0; nt < NT; nt++) {
+      const int f = f0 + 16 * nt;
+      const float wo[4] = {w5[f], w5[f + 1], w5[f + 2], w5[f + 3]};
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) {
+        const float d = ds[16 * mt + lr];
+        float q[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const float zz = z[mt][nt][NH - 1][v], sg = sigm(zz);
+          q[v] = d * wo[v] * sg * (1.0f + zz * (1.0f - sg));
+        }
+        *(uint2 *)(hs + (16 * mt + lr) * HSTR + f) = pack4_bf16(q[0], q[1], q[2], q[3]);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = NMID - 1; k >= 0; k--) {
+      f4 acc[MT][NT];
+      mma(acc);
+      if (k > 0) load_w(g.wb, k - 1);
+      // meanwhile the tile holds the gradient at square layer k's output: its column sums (the first four waves)
+      // and the weight gradient's copy (the others)
+      if (tid < WD) {
+        float a = 0.f;
+#pragma unroll 8
+        for (int r = 0; r < BM; r++) a += bf2f(hs[r * HSTR + tid]);
+        g.part_b[((size_t)k * g.npart + blockIdx.x) * WD + tid] = a;
+      }
+      else {
+        const int f = tid & 255;
+#pragma unroll 1
+        for (int o = (tid >> 8) - 1; o < BM / 8; o += NTHREADS / 256 - 1)
+          *(uint4 *)(g.dzp + k * g.stride + ((size_t)(row0 / 8 + o) * WD + f) * 8) = octet(o, f);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++) {
+        const int f = f0 + 16 * nt;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+          float q[4];
+#pragma unroll
+          for (int v = 0; v < 4; v++) {   // dz_prev = acc silu'(z_prev), silu' = s (1 + z (1 - s))
+            const float zz = z[mt][nt][k][v], s = sigm(zz);
+            q[v] = acc[mt][nt][v] * s * (1.0f + zz * (1.0f - s));
+          }
+          *(uint2 *)(hs + (16 * mt + lr) * HSTR + f) = pack4_bf16(q[0], q[1], q[2], q[3]);
+        }
+      }
+      __syncthreads();
+    }
+    // partials of dW0 = x^T dz1 and db0 = sum_r dz1: part[block][i][c] (i < 8), part[block][8][c]
+    if (tid < WD) {
+      float a[NIN + 1] = {};
+#pragma unroll 4
+      for (int r = 0; r < BM; r++) {
+        const float d = bf2f(hs[r * HSTR + tid]);
+#pragma unroll
+        for (int i = 0; i < NIN; i++) a[i] = fmaf(xs[r * NIN + i], d, a[i]);
+        a[NIN] += d;
+      }
+      for (int i = 0; i <= NIN; i++) g.part_in[((size_t)blockIdx.x * (NIN + 1) + i) * WD + tid] = a[i];
+    }
   }
-  for (int i = 0; i <= NIN; i++) part[((size_t)z * (NIN + 1) + i) * WD + c] = a[i];
 }
 
-__global__ __launch_bounds__(256) void k_gather(const float *__restrict__ Xall, const float *__restrict__ Tall,
-                                                const float *__restrict__ Wall, int n, const DevState *__restrict__ st,
-                                                float *__restrict__ X, float *__restrict__ T, float *__restrict__ Wt)
+// ---------------------------------------------------------------------------------------------
+// gradients of every parameter and their Adam update (Kingma & Ba 2015), one launch.
+// Workgroups 0 .. 255: a 32 x 32 tile of one square layer's dW = h^T dz.  The rows are summed in splits of
+// KSPLIT (each split one chain of MFMAs from zero, as many splits at a time as there are waves), the splits in
+// ascending order through LDS, so that the sum does not depend on the launch.  The operands are read as laid
+// out by k_mlp_rows, 16 bytes per lane with no transposition.  The other workgroups: a thread per remaining
+// parameter, over the row-chunk partials.
+// ---------------------------------------------------------------------------------------------
+struct UpdateArgs {
+  float *p, *m, *v;
+  float *grad;                   // not NULL: write the gradient there and leave the parameters alone
+  uint16_t *wf, *wb;
+  const uint16_t *hp, *dzp;
+  const float *part_in, *part_out, *part_b;
+  DevState *st;
+  size_t stride;
+  int n, npart, npart_alloc;     // rows; row-chunk partials; partials allocated per layer in part_b
+};
+
+constexpr int GT_ = 32;                                 // dW tile edge
+constexpr int TILES = (WD / GT_) * (WD / GT_);          // per layer
+constexpr int NSMALL = (NIN + 1) * WD + NMID * WD + WD + 1;
+constexpr int UPD_BLOCKS = NMID * TILES + (NSMALL + UPD_THREADS - 1) / UPD_THREADS;
+
+__device__ __forceinline__ float adam_update(const UpdateArgs &u, const DevState &a, int64_t i, float g)
 {
-  const int b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= n) return;
-  u32x4 c = {{(uint32_t)st->step, (uint32_t)b, 0u, 0u}};
-  u32x4 r = philox4x32_10(c, st->seed, MLP_KEY1);
-  const uint64_t u = ((uint64_t)r.v[0] << 32) | r.v[1];
-  const int64_t i = (int64_t)(u % (uint64_t)st->ndata);
-  for (int k = 0; k < NIN; k++) X[(size_t)b * NIN + k] = Xall[(size_t)i * NIN + k];
-  T[b] = Tall[i];
-  Wt[b] = Wall[i];
+  // fused products as written, the same on every build
+#pragma clang fp contract(off)
+  const float mi = fmaf(1.0f - a.b1, g, a.b1 * u.m[i]);
+  const float vi = fmaf(a.b2, u.v[i], (1.0f - a.b2) * g * g);
+  u.m[i] = mi;
+  u.v[i] = vi;
+  const float mh = mi / a.c1, vh = vi / a.c2;
+  const float pi = u.p[i] - a.lr * mh / (sqrtf(vh) + a.eps);
+  u.p[i] = pi;
+  return pi;
 }
 
-// Adam (Kingma & Ba 2015) on one contiguous parameter segment; g = sum of nsplit partials
-__global__ __launch_bounds__(256) void k_adam(float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
-                                              uint16_t *__restrict__ pbf, const float *__restrict__ part, int nsplit,
-                                              int64_t count, const DevState *__restrict__ st)
+__global__ __launch_bounds__(UPD_THREADS) void k_mlp_update(UpdateArgs u)
 {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= count) return;
-  float g = 0.f;
-  for (int z = 0; z < nsplit; z++) g += part[(size_t)z * count + i];
-  const int s = st->step;
-  const float frac = st->total > 0 ? fminf((float)s / (float)st->total, 1.0f) : 0.0f;
-  const float lr = st->lr0 * 0.5f * (1.0f + cosf(3.14159265358979f * frac));
-  const float b1 = st->b1, b2 = st->b2;
-  const float mi = b1 * m[i] + (1.0f - b1) * g;
-  const float vi = b2 * v[i] + (1.0f - b2) * g * g;
-  m[i] = mi;
-  v[i] = vi;
-  const float mh = mi / (1.0f - powf(b1, (float)(s + 1))), vh = vi / (1.0f - powf(b2, (float)(s + 1)));
-  const float pi = p[i] - lr * mh / (sqrtf(vh) + st->eps);
-  p[i] = pi;
-  if (pbf) pbf[i] = f2bf(pi);
-}
-
-__global__ __launch_bounds__(256) void k_grad_out(const float *__restrict__ part, int nsplit, int64_t count,
-                                                  float *__restrict__ out)
-{
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= count) return;
-  float g = 0.f;
-  for (int z = 0; z < nsplit; z++) g += part[(size_t)z * count + i];
-  out[i] = g;
-}
-
-__global__ void k_step_done(DevState *st)
-{
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    st->step += 1;
-    st->local += 1;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lr = lane & 15, lg = lane >> 4;
+  const bool update = u.grad == nullptr;
+  if (blockIdx.x < NMID * TILES) {
+    constexpr int NW = UPD_THREADS / 64, PS = GT_ * (GT_ + 1);
+    __shared__ float part[NW * PS];
+    // blocks go to the eight XCDs in turn: two XCDs take one layer each, so that an XCD's L2 reads one layer's
+    // operands (3 MB at 4096 rows) and not all four's
+    static_assert(NMID == 4 && TILES % 2 == 0, "an XCD per half layer");
+    const int xcd = blockIdx.x & 7, layer = xcd >> 1, tile = (xcd & 1) * (TILES / 2) + (blockIdx.x >> 3);
+    const int i0 = (tile / (WD / GT_)) * GT_, j0 = (tile % (WD / GT_)) * GT_;
+    const uint16_t *hp = u.hp + layer * u.stride, *dzp = u.dzp + layer * u.stride;
+    const int ns = (u.n + KSPLIT - 1) / KSPLIT;
+    constexpr int EL = GT_ * GT_ / UPD_THREADS;   // elements per thread
+    float sum[EL] = {};
+    for (int z0 = 0; z0 < ns; z0 += NW) {
+      const int zs = z0 + wv;
+      if (zs < ns) {
+        const int kb = zs * KSPLIT, ke = u.n < kb + KSPLIT ? u.n : kb + KSPLIT;
+        f4 acc[2][2];
+        for (int i = 0; i < 2; i++)
+          for (int j = 0; j < 2; j++) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
+        auto step = [&](int r) {
+          const size_t o = (size_t)(r / 8 + lg) * WD + lr;
+          bf16x8 a[2], b[2];
+          for (int i = 0; i < 2; i++) a[i] = __builtin_bit_cast(bf16x8, *(const uint4 *)(hp + (o + i0 + 16 * i) * 8));
+          for (int j = 0; j < 2; j++) b[j] = __builtin_bit_cast(bf16x8, *(const uint4 *)(dzp + (o + j0 + 16 * j) * 8));
+          for (int i = 0; i < 2; i++)
+            for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        };
+        if (ke - kb == KSPLIT) {   // a whole split: every load in flight before the first product
+#pragma unroll
+          for (int r = 0; r < KSPLIT; r += 32) step(kb + r);
+        }
+        else {
+          for (int r = kb; r < ke; r += 32) step(r);
+        }
+        for (int i = 0; i < 2; i++)
+          for (int j = 0; j < 2; j++)
+            for (int v = 0; v < 4; v++)
+              part[wv * PS + (16 * i + 4 * lg + v) * (GT_ + 1) + 16 * j + lr] = acc[i][j][v];
+      }
+      __syncthreads();
+      const int nz = ns - z0 < NW ? ns - z0 : NW;
+      for (int e = 0; e < EL; e++) {
+        const int el = tid + e * UPD_THREADS, i = el / GT_, j = el % GT_;
+        for (int q = 0; q < nz; q++) sum[e] += part[q * PS + i * (GT_ + 1) + j];
+      }
+      __syncthreads();
+    }
+    const DevState a = *u.st;
+    for (int e = 0; e < EL; e++) {
+      const int el = tid + e * UPD_THREADS, i = i0 + el / GT_, j = j0 + el % GT_;
+      const int64_t idx = OFF_MID + layer * MID_STRIDE + (int64_t)i * WD + j;
+      if (!update) {
+        u.grad[idx] = sum[e];
+        continue;
+      }
+      const uint16_t b = f2bf(adam_update(u, a, idx, sum[e]));
+      u.wf[frag_index(layer, j, i)] = b;
+      u.wb[frag_index(layer, i, j)] = b;
+    }
+    if (update && blockIdx.x == 0 && tid == 0) {
+      u.st->step = u.st->step_b + 1;
+      u.st->local += 1;
+    }
+    return;
   }
+  const int q = (blockIdx.x - NMID * TILES) * UPD_THREADS + tid;
+  if (q >= NSMALL) return;
+  // parameter q of the input layer, the square layers' biases or the output layer: its index, partials and their stride
+  constexpr int NI = (NIN + 1) * WD, NB = NMID * WD;
+  int64_t idx;
+  const float *part;
+  int stride;
+  if (q < NI) {
+    idx = OFF_W0 + q;
+    part = u.part_in + q;
+    stride = NI;
+  }
+  else if (q < NI + NB) {
+    const int k = (q - NI) / WD, c = (q - NI) % WD;
+    idx = OFF_MID + k * MID_STRIDE + (int64_t)WD * WD + c;
+    part = u.part_b + (size_t)k * u.npart_alloc * WD + c;
+    stride = WD;
+  }
+  else {
+    idx = OFF_W5 + (q - NI - NB);
+    part = u.part_out + (q - NI - NB);
+    stride = WD + 1;
+  }
+  float g = 0.f;
+  int z = 0;
+  for (; z + 16 <= u.npart; z += 16) {   // sixteen loads in flight, added in order
+    float q[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) q[e] = part[(size_t)(z + e) * stride];
+#pragma unroll
+    for (int e = 0; e < 16; e++) g += q[e];
+  }
+  for (; z < u.npart; z++) g += part[(size_t)z * stride];
+  if (!update) u.grad[idx] = g;
+  else adam_update(u, *u.st, idx, g);
 }
 
-__global__ __launch_bounds__(256) void k_to_bf16(const float *__restrict__ p, int64_t count, uint16_t *__restrict__ o)
+// the BF16 fragment copies of the square layers, from the FP32 parameters
+__global__ __launch_bounds__(256) void k_pack_weights(const float *__restrict__ p, uint16_t *__restrict__ wf,
+                                                      uint16_t *__restrict__ wb)
 {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < count) o[i] = f2bf(p[i]);
+  const int i = blockIdx.x, j = threadIdx.x, k = blockIdx.y;
+  const uint16_t b = f2bf(p[OFF_MID + k * MID_STRIDE + (int64_t)i * WD + j]);
+  wf[frag_index(k, j, i)] = b;
+  wb[frag_index(k, i, j)] = b;
 }
-
-unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
@@ -310,11 +544,10 @@ struct crime_mlp {
   int max_batch = 0, device = 0;
   hipStream_t stream = nullptr;
   float *p = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr;
-  uint16_t *wbf = nullptr;                  // [NMID][WD][WD]
-  float *X = nullptr, *T = nullptr, *Wt = nullptr, *Y = nullptr, *dy = nullptr;
-  float *Z = nullptr;                       // [NH][max_batch][WD]
-  uint16_t *H = nullptr, *dZ = nullptr;     // [NH][max_batch][WD]
-  float *part_in = nullptr, *part_out = nullptr, *part_w = nullptr, *part_b = nullptr;
+  uint16_t *wf = nullptr, *wb = nullptr;    // BF16 fragments of the square layers, forward and backward order
+  float *X = nullptr, *T = nullptr, *Wt = nullptr, *Y = nullptr;
+  uint16_t *hp = nullptr, *dzp = nullptr;   // [NMID][max_batch * WD] weight-gradient operands (k_mlp_rows)
+  float *part_in = nullptr, *part_out = nullptr, *part_b = nullptr;
   DevState *st = nullptr;
   float *loss = nullptr;
   int loss_cap = 0;
@@ -369,15 +602,14 @@ extern "C" void crime_mlp_destroy(crime_mlp_t *h)
   (void)hipSetDevice(h->device);
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   drop_graph(h);
-  void *bufs[] = {h->p, h->m, h->v, h->grad, h->wbf, h->X, h->T, h->Wt, h->Y, h->dy, h->Z, h->H, h->dZ,
-                  h->part_in, h->part_out, h->part_w, h->part_b, h->st, h->loss, h->Xall, h->Tall, h->Wall};
+  void *bufs[] = {h->p, h->m, h->v, h->grad, h->wf, h->wb, h->X, h->T, h->Wt, h->Y, h->hp, h->dzp,
+                  h->part_in, h->part_out, h->part_b, h->st, h->loss, h->Xall, h->Tall, h->Wall};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
 }
 
-static int nsplit_of(int n) { return (n + KSPLIT - 1) / KSPLIT; }
 static int nred_of(int n) { return (n + RROWS - 1) / RROWS; }
 
 static int create_impl(crime_mlp *h, int max_batch, int device)
@@ -391,24 +623,22 @@ static int create_impl(crime_mlp *h, int max_batch, int device)
   h->device = device;
   MLP_HIP(h, hipSetDevice(device));
   MLP_HIP(h, hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-  const size_t B = (size_t)max_batch, act = (size_t)NH * B * WD;
-  const int ns = nsplit_of(max_batch), nr = nred_of(max_batch);
+  const size_t B = (size_t)max_batch;
+  const int nr = nred_of(max_batch);
   MLP_HIP(h, hipMalloc((void **)&h->p, NPARAM * sizeof(float)));
   MLP_HIP(h, hipMalloc((void **)&h->m, NPARAM * sizeof(float)));
   MLP_HIP(h, hipMalloc((void **)&h->v, NPARAM * sizeof(float)));
   MLP_HIP(h, hipMalloc((void **)&h->grad, NPARAM * sizeof(float)));
-  MLP_HIP(h, hipMalloc((void **)&h->wbf, (size_t)NMID * WD * WD * sizeof(uint16_t)));
+  MLP_HIP(h, hipMalloc((void **)&h->wf, (size_t)NMID * WD * WD * sizeof(uint16_t)));
+  MLP_HIP(h, hipMalloc((void **)&h->wb, (size_t)NMID * WD * WD * sizeof(uint16_t)));
   MLP_HIP(h, hipMalloc((void **)&h->X, B * NIN * sizeof(float)));
   MLP_HIP(h, hipMalloc((void **)&h->T, B * sizeof(float)));
   MLP_HIP(h, hipMalloc((void **)&h->Wt, B * sizeof(float)));
   MLP_HIP(h, hipMalloc((void **)&h->Y, B * sizeof(float)));
-  MLP_HIP(h, hipMalloc((void **)&h->dy, B * sizeof(float)));
-  MLP_HIP(h, hipMalloc((void **)&h->Z, act * sizeof(float)));
-  MLP_HIP(h, hipMalloc((void **)&h->H, act * sizeof(uint16_t)));
-  MLP_HIP(h, hipMalloc((void **)&h->dZ, act * sizeof(uint16_t)));
+  MLP_HIP(h, hipMalloc((void **)&h->hp, NMID * B * WD * sizeof(uint16_t)));
+  MLP_HIP(h, hipMalloc((void **)&h->dzp, NMID * B * WD * sizeof(uint16_t)));
   MLP_HIP(h, hipMalloc((void **)&h->part_in, (size_t)nr * (NIN + 1) * WD * sizeof(float)));
   MLP_HIP(h, hipMalloc((void **)&h->part_out, (size_t)nr * (WD + 1) * sizeof(float)));
-  MLP_HIP(h, hipMalloc((void **)&h->part_w, (size_t)NMID * ns * WD * WD * sizeof(float)));
   MLP_HIP(h, hipMalloc((void **)&h->part_b, (size_t)NMID * nr * WD * sizeof(float)));
   MLP_HIP(h, hipMalloc((void **)&h->st, sizeof(DevState)));
   DevState s{};
@@ -446,9 +676,7 @@ extern "C" int crime_mlp_set_params(crime_mlp_t *h, const float *params)
   MLP_HIP(h, hipMemcpy(h->v, zero.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice));
   DevState s{};
   MLP_HIP(h, hipMemcpy(h->st, &s, sizeof(s), hipMemcpyHostToDevice));
-  for (int k = 0; k < NMID; k++)
-    hipLaunchKernelGGL(k_to_bf16, dim3(nblk((int64_t)WD * WD)), dim3(256), 0, h->stream, h->p + OFF_MID + k * MID_STRIDE,
-                       (int64_t)WD * WD, h->wbf + (size_t)k * WD * WD);
+  hipLaunchKernelGGL(k_pack_weights, dim3(WD, NMID), dim3(WD), 0, h->stream, h->p, h->wf, h->wb);
   MLP_HIP(h, hipGetLastError());
   MLP_HIP(h, hipStreamSynchronize(h->stream));
   return 0;
@@ -464,76 +692,81 @@ extern "C" int crime_mlp_get_params(crime_mlp_t *h, float *params)
   return 0;
 }
 
-// forward over rows [0, n) of h->X
-// forward for rows [0, n) of X (the handle's own input buffer unless given) on stream s (its own unless given)
-static void enqueue_forward(crime_mlp *h, int n, int train, hipStream_t s = nullptr, const float *X = nullptr)
+static RowArgs row_args(crime_mlp *h, int n)
 {
-  const size_t B = (size_t)h->max_batch;
+  RowArgs g{};
+  g.X = h->X;
+  g.T = h->T;
+  g.Wt = h->Wt;
+  g.p = h->p;
+  g.wf = h->wf;
+  g.wb = h->wb;
+  g.Y = h->Y;
+  g.hp = h->hp;
+  g.dzp = h->dzp;
+  g.part_in = h->part_in;
+  g.part_out = h->part_out;
+  g.part_b = h->part_b;
+  g.st = h->st;
+  g.loss = h->loss;
+  g.stride = (size_t)h->max_batch * WD;
+  g.n = n;
+  g.npart = nred_of(h->max_batch);
+  return g;
+}
+
+// forward for rows [0, n) of X (the handle's own input buffer unless given) on stream s (its own unless given).
+// The fewest rows per workgroup that still give every one of the 256 CUs at most one workgroup, as the layers'
+// latency counts there (256 rows: 13 us by 16, 20 us by 32); above that 64 rows, which read the weights less often.
+static void enqueue_forward(crime_mlp *h, int n, hipStream_t s = nullptr, const float *X = nullptr)
+{
   if (!s) s = h->stream;
-  if (!X) X = h->X;
-  hipLaunchKernelGGL(k_in_fwd, dim3(nblk((int64_t)n * WD)), dim3(256), 0, s, X, h->p, n, h->Z, h->H);
-  const dim3 g((n + TM - 1) / TM, WD / TN, 1);
-  for (int k = 0; k < NMID; k++) {
-    EpiFwd e{h->p + OFF_MID + k * MID_STRIDE + (int64_t)WD * WD, h->Z + (size_t)(k + 1) * B * WD,
-             h->H + (size_t)(k + 1) * B * WD};
-    hipLaunchKernelGGL((k_gemm<false, false, EpiFwd>), g, dim3(256), 0, s, h->H + (size_t)k * B * WD, WD,
-                       h->wbf + (size_t)k * WD * WD, WD, n, WD, WD, e);
-  }
-  hipLaunchKernelGGL(k_out, dim3((n + 3) / 4), dim3(256), 0, s, h->H + (size_t)(NH - 1) * B * WD,
-                     h->Z + (size_t)(NH - 1) * B * WD, h->p, h->T, h->Wt, n, train, h->Y, h->dy,
-                     h->dZ + (size_t)(NH - 1) * B * WD, h->st, h->loss);
+  RowArgs g = row_args(h, n);
+  if (X) g.X = X;
+  auto launch = [&](auto bm, auto nt) {
+    constexpr int BM = decltype(bm)::value, NT = decltype(nt)::value;
+    hipLaunchKernelGGL((k_mlp_rows<BM, NT, false>), dim3((n + BM - 1) / BM), dim3(row_threads(NT)), 0, s, g);
+  };
+  using std::integral_constant;
+  if (n <= 256 * 16) launch(integral_constant<int, 16>{}, integral_constant<int, 1>{});
+  else if (n <= 256 * TR) launch(integral_constant<int, TR>{}, integral_constant<int, 1>{});
+  else launch(integral_constant<int, FWD_ROWS>{}, integral_constant<int, 2>{});
 }
 
-// backward for rows [0, n) (n % 64 == 0) into the split partials
-static void enqueue_backward(crime_mlp *h, int n)
+// forward and backward for n rows (n % 64 == 0): of the training set drawn by Philox (gather), or of X, T, Wt
+static void enqueue_rows(crime_mlp *h, int n, bool gather)
 {
-  const size_t B = (size_t)h->max_batch;
-  const int ns = nsplit_of(n), nr = nred_of(n);
-  hipLaunchKernelGGL(k_out_wgrad, dim3(nr), dim3(256), 0, h->stream, h->H + (size_t)(NH - 1) * B * WD, h->dy, n,
-                     h->part_out);
-  for (int k = NMID - 1; k >= 0; k--) {
-    const uint16_t *Hin = h->H + (size_t)k * B * WD;         // input of square layer k
-    const uint16_t *dZo = h->dZ + (size_t)(k + 1) * B * WD;  // gradient at its output
-    EpiPart ep{h->part_w + (size_t)k * nsplit_of(h->max_batch) * WD * WD};
-    hipLaunchKernelGGL((k_gemm<true, false, EpiPart>), dim3(WD / TM, WD / TN, ns), dim3(256), 0, h->stream, Hin, WD,
-                       dZo, WD, WD, n, KSPLIT, ep);
-    hipLaunchKernelGGL(k_colsum, dim3(nr), dim3(256), 0, h->stream, dZo, n,
-                       h->part_b + (size_t)k * nred_of(h->max_batch) * WD);
-    EpiBwd eb{h->Z + (size_t)k * B * WD, h->dZ + (size_t)k * B * WD};
-    hipLaunchKernelGGL((k_gemm<false, true, EpiBwd>), dim3((n + TM - 1) / TM, WD / TN, 1), dim3(256), 0, h->stream,
-                       dZo, WD, h->wbf + (size_t)k * WD * WD, WD, n, WD, WD, eb);
+  RowArgs g = row_args(h, n);
+  if (gather) {
+    g.X = h->Xall;
+    g.T = h->Tall;
+    g.Wt = h->Wall;
+    g.gather = 1;
   }
-  hipLaunchKernelGGL(k_in_wgrad, dim3(nr), dim3(256), 0, h->stream, h->X, h->dZ, n, h->part_in);
+  hipLaunchKernelGGL((k_mlp_rows<TR, 1, true>), dim3(n / TR), dim3(row_threads(1)), 0, h->stream, g);
 }
 
-// segments of the parameter vector and their partials (GEMM splits or row-chunk reductions)
-struct Seg {
-  int64_t off, count;
-  const float *part;
-  bool gemm;
-  int k;   // square layer whose BF16 copy follows the update, or -1
-};
-
-static std::vector<Seg> segments(crime_mlp *h)
+// the gradients of the last enqueue_rows: into grad, or the parameters' Adam update (grad NULL)
+static void enqueue_update(crime_mlp *h, int n, float *grad)
 {
-  const size_t nsm = (size_t)nsplit_of(h->max_batch), nrm = (size_t)nred_of(h->max_batch);
-  std::vector<Seg> s;
-  s.push_back({OFF_W0, (int64_t)(NIN + 1) * WD, h->part_in, false, -1});
-  for (int k = 0; k < NMID; k++) {
-    s.push_back({OFF_MID + k * MID_STRIDE, (int64_t)WD * WD, h->part_w + k * nsm * WD * WD, true, k});
-    s.push_back({OFF_MID + k * MID_STRIDE + (int64_t)WD * WD, WD, h->part_b + k * nrm * WD, false, -1});
-  }
-  s.push_back({OFF_W5, WD + 1, h->part_out, false, -1});
-  return s;
-}
-
-static void enqueue_adam(crime_mlp *h, int n)
-{
-  for (const Seg &g : segments(h))
-    hipLaunchKernelGGL(k_adam, dim3(nblk(g.count)), dim3(256), 0, h->stream, h->p + g.off, h->m + g.off, h->v + g.off,
-                       g.k >= 0 ? h->wbf + (size_t)g.k * WD * WD : (uint16_t *)nullptr, g.part,
-                       g.gemm ? nsplit_of(n) : nred_of(n), g.count, h->st);
-  hipLaunchKernelGGL(k_step_done, dim3(1), dim3(64), 0, h->stream, h->st);
+  UpdateArgs u{};
+  u.p = h->p;
+  u.m = h->m;
+  u.v = h->v;
+  u.grad = grad;
+  u.wf = h->wf;
+  u.wb = h->wb;
+  u.hp = h->hp;
+  u.dzp = h->dzp;
+  u.part_in = h->part_in;
+  u.part_out = h->part_out;
+  u.part_b = h->part_b;
+  u.st = h->st;
+  u.stride = (size_t)h->max_batch * WD;
+  u.n = n;
+  u.npart = nred_of(n);
+  u.npart_alloc = nred_of(h->max_batch);
+  hipLaunchKernelGGL(k_mlp_update, dim3(UPD_BLOCKS), dim3(UPD_THREADS), 0, h->stream, u);
 }
 
 static int ensure_loss(crime_mlp *h, int n)
@@ -553,12 +786,10 @@ extern "C" int crime_mlp_forward(crime_mlp_t *h, int64_t n, const float *x, floa
   if (!h) return mlp_error(nullptr, CRIME_GH_EINVAL, "handle is NULL");
   if (n < 1 || !x || !y) return mlp_error(h, CRIME_GH_EINVAL, "need n >= 1 and non-NULL x, y");
   MLP_HIP(h, hipSetDevice(h->device));
-  int rc = ensure_loss(h, 1);
-  if (rc) return rc;
   for (int64_t i0 = 0; i0 < n; i0 += h->max_batch) {
     const int c = (int)(n - i0 < h->max_batch ? n - i0 : h->max_batch);
     MLP_HIP(h, hipMemcpyAsync(h->X, x + i0 * NIN, (size_t)c * NIN * sizeof(float), hipMemcpyHostToDevice, h->stream));
-    enqueue_forward(h, c, 0);
+    enqueue_forward(h, c);
     MLP_HIP(h, hipGetLastError());
     MLP_HIP(h, hipMemcpyAsync(y + i0, h->Y, (size_t)c * sizeof(float), hipMemcpyDeviceToHost, h->stream));
   }
@@ -586,11 +817,7 @@ extern "C" int crime_mlp_forward_mean(crime_mlp_t *const *hs, int nh, int64_t n,
     batch = std::min(batch, hs[k]->max_batch);
   }
   MLP_HIP(h0, hipSetDevice(h0->device));
-  for (int k = 0; k < nh; k++) {
-    int rc = ensure_loss(hs[k], 1);
-    if (rc) return rc;
-    MLP_HIP(h0, hipStreamSynchronize(hs[k]->stream));  // no pending work of a handle on its buffers
-  }
+  for (int k = 0; k < nh; k++) MLP_HIP(h0, hipStreamSynchronize(hs[k]->stream));  // no pending work on its buffers
   // every network reads the first handle's input buffer on the first handle's stream; the mean collects in
   // its target buffer (scratch outside a training step)
   hipStream_t s = h0->stream;
@@ -599,7 +826,7 @@ extern "C" int crime_mlp_forward_mean(crime_mlp_t *const *hs, int nh, int64_t n,
     const int c = (int)(n - i0 < batch ? n - i0 : batch);
     MLP_HIP(h0, hipMemcpyAsync(h0->X, x + i0 * NIN, (size_t)c * NIN * sizeof(float), hipMemcpyHostToDevice, s));
     for (int k = 0; k < nh; k++) {
-      enqueue_forward(hs[k], c, 0, s, h0->X);
+      enqueue_forward(hs[k], c, s, h0->X);
       hipLaunchKernelGGL(k_acc_rows, dim3((c + 255) / 256), dim3(256), 0, s, h0->T, hs[k]->Y, c, w, k == 0);
     }
     MLP_HIP(h0, hipGetLastError());
@@ -634,11 +861,8 @@ extern "C" int crime_mlp_loss_grad(crime_mlp_t *h, int n, const float *x, const 
     std::vector<float> ones((size_t)n, 1.0f);
     MLP_HIP(h, hipMemcpy(h->Wt, ones.data(), (size_t)n * sizeof(float), hipMemcpyHostToDevice));
   }
-  enqueue_forward(h, n, 1);
-  enqueue_backward(h, n);
-  for (const Seg &g : segments(h))
-    hipLaunchKernelGGL(k_grad_out, dim3(nblk(g.count)), dim3(256), 0, h->stream, g.part,
-                       g.gemm ? nsplit_of(n) : nred_of(n), g.count, h->grad + g.off);
+  enqueue_rows(h, n, false);
+  enqueue_update(h, n, h->grad);
   MLP_HIP(h, hipGetLastError());
   MLP_HIP(h, hipStreamSynchronize(h->stream));
   float l = 0;
@@ -710,11 +934,8 @@ extern "C" int crime_mlp_train(crime_mlp_t *h, int steps, int batch, float lr0, 
   MLP_HIP(h, hipMemset(h->loss, 0, (size_t)steps * sizeof(float)));
   if (!h->use_graph) {
     for (int i = 0; i < steps; i++) {
-      hipLaunchKernelGGL(k_gather, dim3(nblk(batch)), dim3(256), 0, h->stream, h->Xall, h->Tall, h->Wall, batch, h->st,
-                         h->X, h->T, h->Wt);
-      enqueue_forward(h, batch, 1);
-      enqueue_backward(h, batch);
-      enqueue_adam(h, batch);
+      enqueue_rows(h, batch, true);
+      enqueue_update(h, batch, nullptr);
       MLP_HIP(h, hipGetLastError());
     }
     MLP_HIP(h, hipStreamSynchronize(h->stream));
@@ -724,11 +945,8 @@ extern "C" int crime_mlp_train(crime_mlp_t *h, int steps, int batch, float lr0, 
   if (h->exec && h->graph_batch != batch) drop_graph(h);
   if (!h->exec) {
     MLP_HIP(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    hipLaunchKernelGGL(k_gather, dim3(nblk(batch)), dim3(256), 0, h->stream, h->Xall, h->Tall, h->Wall, batch, h->st,
-                       h->X, h->T, h->Wt);
-    enqueue_forward(h, batch, 1);
-    enqueue_backward(h, batch);
-    enqueue_adam(h, batch);
+    enqueue_rows(h, batch, true);
+    enqueue_update(h, batch, nullptr);
     hipError_t e = hipStreamEndCapture(h->stream, &h->graph);
     if (e != hipSuccess) {
       h->graph = nullptr;
