@@ -615,7 +615,29 @@ extern "C" int crime_sht_cls_pairs_device(crime_sht_t *p, int nmaps, const void 
   for (int i = 0; i < 2 * npairs; i++)
     if (pairs[i] < 0 || pairs[i] >= nmaps) return sht_error(p, CRIME_GH_EINVAL, "pair index %d outside [0, %d)", pairs[i], nmaps);
   SHT_HIP(p, hipSetDevice(p->device));
-  int rc = analyse(p, nmaps, d_maps, maps_fp64);
+  // only the maps that some pair names are transformed, in ascending order (a training mock's 16 pairs name 16 of
+  // its 64 channels); the pairs then go by the position in that list
+  std::vector<int32_t> slot, used, pr(pairs, pairs + 2 * (size_t)npairs);
+  if (nmaps >= 1 && nmaps <= p->max_maps && d_maps) {
+    slot.assign(nmaps, -1);
+    for (int32_t c : pr) slot[c] = 0;
+    for (int c = 0; c < nmaps; c++)
+      if (slot[c] == 0) {
+        slot[c] = (int32_t)used.size();
+        used.push_back(c);
+      }
+    for (int32_t &c : pr) c = slot[c];
+  }
+  int rc;
+  if (used.empty() || (int)used.size() == nmaps) {
+    rc = analyse(p, nmaps, d_maps, maps_fp64);
+  }
+  else {
+    std::vector<const void *> at(used.size());
+    const size_t bytes = (size_t)p->npix * (maps_fp64 ? sizeof(double) : sizeof(float));
+    for (size_t i = 0; i < used.size(); i++) at[i] = (const char *)d_maps + used[i] * bytes;
+    rc = analyse_sets(p, (int)used.size(), at.data(), 1, maps_fp64);
+  }
   if (rc) return rc;
   const size_t n = (size_t)npairs * (p->lmax + 1);
   const size_t need = n + (size_t)npairs;  // spectra, then the pair list (as int32 pairs in doubles' room)
@@ -627,7 +649,7 @@ extern "C" int crime_sht_cls_pairs_device(crime_sht_t *p, int nmaps, const void 
     p->cls_cap = need;
   }
   int *d_pairs = (int *)(p->d_cls + n);
-  SHT_HIP(p, hipMemcpyAsync(d_pairs, pairs, 2 * (size_t)npairs * sizeof(int32_t), hipMemcpyHostToDevice, p->stream));
+  SHT_HIP(p, hipMemcpyAsync(d_pairs, pr.data(), 2 * (size_t)npairs * sizeof(int32_t), hipMemcpyHostToDevice, p->stream));
   SHT_HIP(p, launch_cls_pairs(p->d_alm, p->lmax, p->ldo, npairs, d_pairs, p->d_cls, p->stream));
   rc = finish(p, true);
   if (rc) return rc;
