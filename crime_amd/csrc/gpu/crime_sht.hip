@@ -26,7 +26,7 @@ constexpr int BLU_MAX_M = 8192;   // largest compiled Bluestein convolution
 
 struct Chunk {
   int m0, m1;        // [m0, m1)
-  int tile0, ntile;  // slice of the analysis tile list
+  XcdRuns tiles;     // the XCDs' runs of the analysis tile list
   int syn0, nsyn;    // slice of the synthesis tile list
 };
 
@@ -337,7 +337,7 @@ static int create_impl(crime_sht *p, int64_t nside, int lmax, int max_maps, int 
   for (int m = 0; m <= lmax;) {
     Chunk c;
     c.m0 = m;
-    c.tile0 = (int)tiles.size();
+    const int tile0 = (int)tiles.size();
     c.syn0 = (int)syn_tiles.size();
     size_t rows = 0;
     while (m <= lmax && (rows == 0 || (rows + (size_t)(lmax - m + 1)) * row_bytes <= LAMBDA_BUDGET)) {
@@ -345,14 +345,21 @@ static int create_impl(crime_sht *p, int64_t nside, int lmax, int max_maps, int 
       const int L = lmax - m + 1;
       for (int par = 0; par < 2; par++) {
         const int nr = (L - par + 1) / 2;
-        for (int rt = 0; rt * ALM_ROWS < nr; rt++) tiles.push_back(make_int4(m, par, rt, nr));
+        for (int r0 = 0; r0 < nr; r0 += ALM_ROWS)
+          tiles.push_back(make_int4(m, par, nr - r0 > ALM_ROWS / 2 ? r0 | ALM_TALL : r0, nr));
         // synthesis: every ring tile, also when this parity has no rows (its spectra are zero)
         for (int rt = 0; rt < nringtiles; rt++) syn_tiles.push_back(make_int4(m, par, rt, nr));
       }
       m++;
     }
     c.m1 = m;
-    c.ntile = (int)tiles.size() - c.tile0;
+    // the XCDs' runs of equal work: a tall tile costs two short ones
+    int64_t total = 0, at = 0;
+    for (size_t i = tile0; i < tiles.size(); i++) total += tiles[i].z & ALM_TALL ? 2 : 1;
+    for (int x = 0, i = tile0; x <= 8; x++) {
+      while (i < (int)tiles.size() && at < total * x / 8) at += tiles[i++].z & ALM_TALL ? 2 : 1;
+      c.tiles.start[x] = x == 8 ? (int)tiles.size() : i;
+    }
     c.nsyn = (int)syn_tiles.size() - c.syn0;
     if (rows > max_chunk_rows) max_chunk_rows = rows;
     p->chunks.push_back(c);
@@ -479,7 +486,7 @@ static int analyse_sets(crime_sht *p, int nsets, const void *const *d_maps, int 
       SHT_HIP(p, launch_legendre(p->d_coef, p->d_off, c.m0, c.m1, p->lmax, p->d_z, p->d_st, p->R, p->RP, p->d_lam,
                                  p->stream));
     SHT_HIP(p, hipEventRecord(ev[2 + 2 * i], p->stream));
-    SHT_HIP(p, launch_alm_gemm(p->d_lam, p->d_G, p->d_tiles + c.tile0, c.ntile, p->d_off, c.m0, p->lmax, p->RP,
+    SHT_HIP(p, launch_alm_gemm(p->d_lam, p->d_G, p->d_tiles, c.tiles, p->d_off, c.m0, p->lmax, p->RP,
                                p->ldg, 2 * nmaps, p->d_alm, p->ldo, p->stream));
     SHT_HIP(p, hipEventRecord(ev[3 + 2 * i], p->stream));
   }

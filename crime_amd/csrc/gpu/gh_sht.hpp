@@ -53,14 +53,16 @@ hipError_t launch_blu_setup(int M, const ShtRing *rings, int r0, int nr, const i
                             const int64_t *boff, void *B, const void *tw, hipStream_t s);
 hipError_t launch_legendre(const double2 *coef, const int64_t *off, int m0, int m1, int lmax, const double *zs,
                            const double *sts, int R, int RP, double *lam, hipStream_t s);
-// tiles: (m, parity, row tile, rows of that parity)
-// rows (l values of one parity) per alm GEMM tile
-#ifndef CRIME_ALM_ROWS
-#define CRIME_ALM_ROWS 128
-#endif
-constexpr int ALM_ROWS = CRIME_ALM_ROWS;
-hipError_t launch_alm_gemm(const double *lam, const double *G, const int4 *tiles, int ntiles, const int64_t *off,
-                           int m0, int lmax, int RP, int ldg, int ncols, double *alm, int ldo, hipStream_t s);
+// runs of consecutive blocks or tiles, one per XCD: [start[x], start[x + 1])
+struct XcdRuns {
+  int start[9];
+};
+// analysis tiles: (m, parity, first row | ALM_TALL for a tile of ALM_ROWS rows, else half as many; rows of that
+// parity), rows being the l values of one parity
+constexpr int ALM_ROWS = 128, ALM_TALL = 1 << 30;
+hipError_t launch_alm_gemm(const double *lam, const double *G, const int4 *tiles, const XcdRuns &xr,
+                           const int64_t *off, int m0, int lmax, int RP, int ldg, int ncols, double *alm, int ldo,
+                           hipStream_t s);
 // cross spectra within each of nsets consecutive sets of mps maps: cls[set][a][b][l]
 hipError_t launch_cls_sets(const double *alm, int lmax, int nsets, int mps, int ldo, double *cls, hipStream_t s);
 hipError_t launch_cls(const double *alm, int lmax, int nmaps, int ldo, int cross, double *cls, hipStream_t s);

@@ -14,6 +14,7 @@
 #include "gh_sht.hpp"
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace crime {
@@ -523,95 +524,141 @@ __global__ __launch_bounds__(256) void k_legendre(const double2 *__restrict__ co
 // j + 16 k for B[k][j]; D[i][j] in lane j + 16 (i % 4), element i / 4 -- measured on gfx950).
 // ---------------------------------------------------------------------------------------------
 typedef double dbl4 __attribute__((ext_vector_type(4)));
+typedef double dbl2 __attribute__((ext_vector_type(2)));
 
 constexpr int GT = 64, GK = 16;
 static_assert(GK == 16, "a GEMM k-step is one 16-ring block of G");
-static_assert(ALM_ROWS == 64 || ALM_ROWS == 128, "alm tiles of 64 or 128 rows");
+static_assert(ALM_ROWS == 128, "alm tiles of 128 or 64 rows");
 #ifndef CRIME_SYN_COLS
 #define CRIME_SYN_COLS 64
 #endif
 constexpr int SYN_COLS = CRIME_SYN_COLS;   // columns per synthesis GEMM tile (64 or 128)
 static_assert(SYN_COLS == 64 || SYN_COLS == 128, "synthesis tiles of 64 or 128 columns");
 
-// alm[l][col] = sum_r lambda_lm(r) G[r][col] per (m, parity): a workgroup computes ALM_ROWS x GT of
-// it, its 4 waves 2 x 2 blocks of (ALM_ROWS / 2) x 32 with 16x16x4 FP64 MFMAs.
-__global__ __launch_bounds__(256) void k_alm_gemm(const double *__restrict__ lam, const double *__restrict__ G,
-                                                  const int4 *__restrict__ tiles, int ntiles, int ncoltiles,
-                                                  int tiles_per_xcd, const int64_t *__restrict__ off, int m0,
-                                                  int lmax, int RP, int ldg, int ncols, double *__restrict__ alm,
-                                                  int ldo)
+// alm[l][col] = sum_r lambda_lm(r) G[r][col] per (m, parity): a workgroup computes 64 NI rows x 16 C columns of
+// it, each of its 4 waves 16 NI rows of every column with 16x16x4 FP64 MFMAs.  tile.z holds the first row and, in
+// bit 30, NI - 1: a unit's rows come in tiles of 128, the last 64 or fewer in a tile of half the height, and a wave
+// whose rows all lie beyond the unit leaves the matrix unit to the others.  C (columns in blocks of 16, at most 6)
+// is the width that covers the call's columns with the least padding (alm_col_blocks).
+// A wave's Legendre rows are its own, so they go from memory to registers, 32 consecutive bytes per lane: lane
+// group g = lane / 16 holds rings 4 g .. 4 g + 3 of a 16-ring step, and the four MFMAs of the step take ring 4 g + q
+// of each group from both operands.  Only G's 16 rows pass through LDS, in two buffers with one barrier per step.
+// Rows and columns out of range are read from an in-range address and not stored: the loop has no selects.
+// What bounds it: the FP64 matrix rate, with three waves per SIMD to cover the loads.  200 maps at Nside 512: 15.6 ms, 62 TFLOP/s of the
+// 72.8 that a large library product reaches, against 18.9 ms for fixed tiles of 128 x 64 through LDS, whose padding
+// (17% of the rows, 12% of the columns) was a quarter of their products.
+template <int NI, int C>
+__device__ __forceinline__ void alm_gemm_tile(const double *__restrict__ lam, const double *__restrict__ G, int m,
+                                              int par, int row0, int nrows, int col0, const int64_t *__restrict__ off,
+                                              int m0, int lmax, int RP, int ldg, int ncols,
+                                              double *__restrict__ alm, int ldo, double *Bs_)
 {
-  constexpr int RW = ALM_ROWS / 2, NI = RW / 16;     // rows per wave, MFMA row blocks per wave
-  constexpr int AL = ALM_ROWS * GK / 256;            // A doubles loaded per thread
-  // XCD-aware order: consecutive logical tiles (which share Legendre rows) stay on one XCD's L2
-  const int b = blockIdx.x;
-  const int logical = (b % 8) * tiles_per_xcd + b / 8;
-  if (logical >= ntiles * ncoltiles) return;
-  const int4 tl = tiles[logical / ncoltiles];
-  const int ct = logical % ncoltiles;
-  const int m = tl.x, par = tl.y, rt = tl.z, nrows = tl.w;
-  __shared__ double As[ALM_ROWS][GK + 1];
-  __shared__ double Bs[GK][GT + 2];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int row0 = rt * ALM_ROWS, col0 = ct * GT;
+  constexpr int BS = 16 * C + 2, BUF = GK * BS + 2;  // LDS row stride; a buffer and a slot that nothing reads
+  constexpr int NB = (8 * C * GK + 255) / 256;       // B double2 loaded per thread
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
   const double *lrow = lam + (size_t)(off[m] - off[m0]) * RP;   // row (l - m) of this m
-
-  dbl4 acc[NI][2];
-  for (int i = 0; i < NI; i++)
-    for (int j = 0; j < 2; j++) acc[i][j] = (dbl4){0, 0, 0, 0};
-  const int ar = tid / (GK / AL), ak = (tid % (GK / AL)) * AL;   // A loads: row ar, AL rings
-  const int bk = tid >> 4, bc = (tid & 15) * 4;                    // B loads: ring bk, 4 columns
-  // Operands out of range are read from an in-range address and zeroed by a select, so the loop
-  // has no divergent branches (they would make the compiler shuttle the accumulators between
-  // AGPRs and VGPRs every step).  ncols is even and col0 + bc a multiple of 4, so each double2
-  // of B is wholly in range or wholly out.
-  const bool arow_ok = row0 + ar < nrows;
-  const double *ap = lrow + (size_t)(par + 2 * (arow_ok ? row0 + ar : 0)) * RP + ak;
-  const bool b0_ok = col0 + bc < ncols, b1_ok = col0 + bc + 2 < ncols;
-  const int bcol0 = b0_ok ? col0 + bc : 0, bcol1 = b1_ok ? col0 + bc + 2 : 0;
-  const int wr = (wv >> 1) * RW, wc = (wv & 1) * 32;
-  // the next k-step's operands are fetched into registers while this one's MFMAs run
-  double2 ra[AL / 2], rb0, rb1;
-  auto fetch = [&](int k0) {
-    for (int e = 0; e < AL / 2; e++) ra[e] = *(const double2 *)(ap + k0 + 2 * e);
-    const double *bp = G + g_block(k0 >> 4, m, par, lmax, ldg) + (size_t)bk * ldg;
-    rb0 = *(const double2 *)(bp + bcol0);
-    rb1 = *(const double2 *)(bp + bcol1);
+  const double *ap[NI];
+#pragma unroll
+  for (int i = 0; i < NI; i++) {
+    const int row = row0 + 16 * (NI * wv + i) + lr;
+    ap[i] = lrow + (size_t)(par + 2 * (row < nrows ? row : row0)) * RP + 4 * lg;
+  }
+  int bsrc[NB], bdst[NB];
+#pragma unroll
+  for (int e = 0; e < NB; e++) {
+    const int q = tid + 256 * e, k = q / (8 * C), c = col0 + 2 * (q % (8 * C));
+    const bool in = q < 8 * C * GK;
+    bsrc[e] = (in ? k : 0) * ldg + (c < ncols ? c : 0);
+    bdst[e] = in ? k * BS + c - col0 : GK * BS;
+  }
+  dbl2 ra[NI][2], rb[NB];
+  auto fetch = [&](int k0) __attribute__((always_inline)) {
+    const double *bp = G + g_block(k0 >> 4, m, par, lmax, ldg);
+#pragma unroll
+    for (int e = 0; e < NB; e++) rb[e] = *(const dbl2 *)(bp + bsrc[e]);
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      ra[i][0] = *(const dbl2 *)(ap[i] + k0);
+      ra[i][1] = *(const dbl2 *)(ap[i] + k0 + 2);
+    }
+  };
+  // rows of the step in LDS buffer b: written, and the next step's operands (none after the last: its own again,
+  // so that the loop has no branch) on their way
+  auto stage = [&](int k0, int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < NB; e++) *(dbl2 *)(Bs_ + b + bdst[e]) = rb[e];
+    __syncthreads();
+    fetch(k0 + GK < RP ? k0 + GK : k0);
   };
   fetch(0);
-  for (int k0 = 0; k0 < RP; k0 += GK) {
-    for (int e = 0; e < AL / 2; e++) {
-      As[ar][ak + 2 * e] = arow_ok ? ra[e].x : 0.0;
-      As[ar][ak + 2 * e + 1] = arow_ok ? ra[e].y : 0.0;
-    }
-    Bs[bk][bc] = b0_ok ? rb0.x : 0.0;
-    Bs[bk][bc + 1] = b0_ok ? rb0.y : 0.0;
-    Bs[bk][bc + 2] = b1_ok ? rb1.x : 0.0;
-    Bs[bk][bc + 3] = b1_ok ? rb1.y : 0.0;
-    __syncthreads();
-    fetch(k0 + GK < RP ? k0 + GK : k0);   // the last step refetches its own operands: no branch
+  if (row0 + 16 * NI * wv >= nrows) {   // a wave without rows: the same barriers, no products
+    for (int k0 = 0, b = 0; k0 < RP; k0 += GK, b = BUF - b) stage(k0, b);
+    return;
+  }
+  dbl4 acc[NI][C];
 #pragma unroll
-    for (int kk = 0; kk < GK; kk += 4) {
-      double af[NI], bf[2];
-      for (int i = 0; i < NI; i++) af[i] = As[wr + 16 * i + (lane & 15)][kk + (lane >> 4)];
-      for (int j = 0; j < 2; j++) bf[j] = Bs[kk + (lane >> 4)][wc + 16 * j + (lane & 15)];
-      for (int i = 0; i < NI; i++)
-        for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
+  for (int i = 0; i < NI; i++)
+#pragma unroll
+    for (int j = 0; j < C; j++) acc[i][j] = (dbl4){0, 0, 0, 0};
+  for (int k0 = 0, b = 0; k0 < RP; k0 += GK, b = BUF - b) {
+    double af[NI][4];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      af[i][0] = ra[i][0].x;
+      af[i][1] = ra[i][0].y;
+      af[i][2] = ra[i][1].x;
+      af[i][3] = ra[i][1].y;
     }
-    __syncthreads();
+    stage(k0, b);
+    const double *bl = Bs_ + b + 4 * lg * BS + lr;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      double bf[C];
+#pragma unroll
+      for (int j = 0; j < C; j++) bf[j] = bl[q * BS + 16 * j];
+#pragma unroll
+      for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int j = 0; j < C; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i][q], bf[j], acc[i][j], 0, 0, 0);
+    }
   }
   const int64_t base_idx = (int64_t)m * lmax - (int64_t)m * (m - 1) / 2;   // he_indexlm(l, m) - l
+#pragma unroll
   for (int i = 0; i < NI; i++)
-    for (int j = 0; j < 2; j++)
+#pragma unroll
+    for (int j = 0; j < C; j++)
+#pragma unroll
       for (int v = 0; v < 4; v++) {
-        const int row = row0 + wr + 16 * i + (lane >> 4) + 4 * v;
-        const int col = col0 + wc + 16 * j + (lane & 15);
+        const int row = row0 + 16 * (NI * wv + i) + lg + 4 * v;
+        const int col = col0 + 16 * j + lr;
         if (row < nrows && col < ncols) {
           const int l = m + par + 2 * row;
           const int64_t idx = m > 0 ? base_idx + l : l;
           alm[(size_t)idx * ldo + col] = acc[i][j][v];
         }
       }
+}
+
+template <int C>
+__global__ __launch_bounds__(256, 3) void k_alm_gemm(const double *__restrict__ lam, const double *__restrict__ G,
+                                                  const int4 *__restrict__ tiles, int ncoltiles, XcdRuns xr,
+                                                  const int64_t *__restrict__ off, int m0, int lmax, int RP, int ldg,
+                                                  int ncols, double *__restrict__ alm, int ldo)
+{
+  __shared__ __align__(16) double Bs[2 * (GK * (16 * C + 2) + 2)];
+  // each XCD takes one contiguous run of tiles (which share Legendre rows and ring spectra in its L2), cut at
+  // equal work
+  const int x = blockIdx.x & 7, q = blockIdx.x >> 3;
+  const int tile = xr.start[x] + q / ncoltiles;
+  if (tile >= xr.start[x + 1]) return;
+  const int4 tl = tiles[tile];
+  const int col0 = (q % ncoltiles) * 16 * C, row0 = tl.z & ~ALM_TALL;
+  if (tl.z & ALM_TALL)
+    alm_gemm_tile<2, C>(lam, G, tl.x, tl.y, row0, tl.w, col0, off, m0, lmax, RP, ldg, ncols, alm, ldo, Bs);
+  else
+    alm_gemm_tile<1, C>(lam, G, tl.x, tl.y, row0, tl.w, col0, off, m0, lmax, RP, ldg, ncols, alm, ldo, Bs);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -625,10 +672,6 @@ __global__ __launch_bounds__(256) void k_alm_gemm(const double *__restrict__ lam
 // blocks of one XCD take consecutive l of one tile and the [set][a][b][l] stores of neighbouring l meet
 // in that XCD's L2.  A block's work grows with l, so the host cuts the runs at equal work, not at equal
 // block counts (launch_cls_sets).
-struct XcdRuns {
-  int start[9];
-};
-
 __global__ __launch_bounds__(256) void k_cls_cross(const double *__restrict__ alm, int lmax, int mps, int ldo,
                                                    int ntile, XcdRuns xr, double *__restrict__ cls)
 {
@@ -700,6 +743,101 @@ __global__ __launch_bounds__(256) void k_cls_cross(const double *__restrict__ al
           if (ta != tb) out[((size_t)b * mps + a) * nl + l] = c;
         }
       }
+}
+
+// The same for 65 to 256 maps per set, one workgroup per (set, l): its 8 waves hold every 16 x 16 block of the upper
+// triangle of C_l (NB (NB + 1) / 2 of them), so each row of alms is read once, and no block is computed twice or for
+// maps that do not exist.  8 m (16 k) pass through LDS at a time, in two buffers; the factor 2 of m > 0 is applied
+// to the sum, m = 0 entering with 1/2 (both exact).  Blocks run by falling l in groups of 16 consecutive l per XCD,
+// whose stores ([a][b][l]) then meet in one L2.
+// What bounds it: the FP64 matrix rate and the 8-byte stores.  200 maps at lmax 1535: 2.3 ms against 5.3
+// ms for pairs of 64 x 64 tiles, which read every row seven times and computed 160 blocks of 16 x 16 where 91 are needed.
+constexpr int CLS_THREADS = 512;
+template <int NB>
+__global__ __launch_bounds__(CLS_THREADS) void k_cls_triangle(const double *__restrict__ alm, int lmax, int mps, int ldo,
+                                                              double *__restrict__ cls)
+{
+  constexpr int NP = NB * (NB + 1) / 2, PW = (NP + 7) / 8;   // blocks, and blocks per wave
+  constexpr int MC = 8, NC = 16 * NB, XS = NC + 2, BUF = 2 * MC * XS;
+  constexpr int NL = (MC * NC + CLS_THREADS - 1) / CLS_THREADS;
+  __shared__ __align__(16) double Xs[2 * BUF];
+  const int nl = lmax + 1, ng = (nl + 15) / 16;
+  // group g of 16 l (from the largest) goes to XCD g mod 8; a set's groups follow the previous set's
+  const int x = blockIdx.x & 7, q = blockIdx.x >> 3, per = (ng + 7) / 8;
+  const int set = q / (per * 16), g = (q % (per * 16)) / 16 * 8 + x, l = lmax - (16 * g + (q & 15));
+  if (g >= ng || l < 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const double *base = alm + (size_t)2 * set * mps;
+  // this wave's blocks (bi <= bj), in rows of the triangle
+  int bi[PW], bj[PW];
+#pragma unroll
+  for (int p = 0; p < PW; p++) {
+    int t = wv * PW + p < NP ? wv * PW + p : NP - 1, i = 0;
+    while (t >= NB - i) {
+      t -= NB - i;
+      i++;
+    }
+    bi[p] = i;
+    bj[p] = i + t;
+  }
+  int lm[NL], lc[NL];
+#pragma unroll
+  for (int e = 0; e < NL; e++) {
+    const int it = tid + CLS_THREADS * e;
+    lm[e] = it < MC * NC ? it / NC : -1;
+    lc[e] = it % NC;
+  }
+  dbl2 r[NL];
+  auto fetch = [&](int mc) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < NL; e++) {
+      const int m = mc + (lm[e] < 0 ? 0 : lm[e]), mm = m <= l ? m : 0;
+      const int64_t idx = mm > 0 ? l + (int64_t)mm * lmax - (int64_t)mm * (mm - 1) / 2 : l;
+      const dbl2 v = *(const dbl2 *)(base + (size_t)idx * ldo + 2 * (lc[e] < mps ? lc[e] : 0));
+      r[e] = m <= l ? v : (dbl2){0.0, 0.0};
+    }
+  };
+  dbl4 acc[PW];
+#pragma unroll
+  for (int p = 0; p < PW; p++) acc[p] = (dbl4){0, 0, 0, 0};
+  fetch(0);
+  for (int mc = 0, b = 0; mc <= l; mc += MC, b = BUF - b) {
+#pragma unroll
+    for (int e = 0; e < NL; e++)
+      if (lm[e] >= 0) {
+        Xs[b + 2 * lm[e] * XS + lc[e]] = r[e].x;
+        Xs[b + (2 * lm[e] + 1) * XS + lc[e]] = r[e].y;
+      }
+    __syncthreads();
+    fetch(mc + MC <= l ? mc + MC : mc);
+    const double *xl = Xs + b + lg * XS + lr;
+#pragma unroll
+    for (int kk = 0; kk < 2 * MC; kk += 4) {
+      // k = kk + lg; k < 2 is m = 0
+      const double w = mc + kk == 0 && lg < 2 ? 0.5 : 1.0;
+#pragma unroll
+      for (int p = 0; p < PW; p++)
+        acc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(w * xl[kk * XS + 16 * bi[p]], xl[kk * XS + 16 * bj[p]], acc[p], 0,
+                                                      0, 0);
+    }
+  }
+  const double inv = 2.0 / (2.0 * l + 1.0);
+  double *out = cls + (size_t)set * mps * mps * nl + l;
+#pragma unroll
+  for (int p = 0; p < PW; p++) {
+    if (wv * PW + p >= NP) break;
+    const int cb = 16 * bj[p] + lr;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int ca = 16 * bi[p] + lg + 4 * v;
+      if (ca < mps && cb < mps) {
+        const double c = acc[p][v] * inv;
+        out[((size_t)ca * mps + cb) * nl] = c;
+        if (bi[p] != bj[p]) out[((size_t)cb * mps + ca) * nl] = c;
+      }
+    }
+  }
 }
 
 __global__ __launch_bounds__(256) void k_cls_auto(const double *__restrict__ alm, int lmax, int nmaps, int ldo,
@@ -1073,14 +1211,42 @@ hipError_t launch_legendre(const double2 *coef, const int64_t *off, int m0, int 
   return hipGetLastError();
 }
 
-hipError_t launch_alm_gemm(const double *lam, const double *G, const int4 *tiles, int ntiles, const int64_t *off,
-                           int m0, int lmax, int RP, int ldg, int ncols, double *alm, int ldo, hipStream_t s)
+// Column blocks (of 16) per alm GEMM tile: the width in [1, 6] that covers the columns with the fewest padded
+// blocks, each tile counted half a block more for the Legendre rows that it reads again
+static int alm_col_blocks(int ncols)
 {
-  const int ncoltiles = (ncols + GT - 1) / GT;
-  const long total = (long)ntiles * ncoltiles;
-  const int per_xcd = (int)((total + 7) / 8);
-  hipLaunchKernelGGL(k_alm_gemm, dim3(8 * per_xcd), dim3(256), 0, s, lam, G, tiles, ntiles, ncoltiles, per_xcd, off,
-                     m0, lmax, RP, ldg, ncols, alm, ldo);
+  const int nb = (ncols + 15) / 16;
+  int best = 1;
+  double cost = 1e300;
+  for (int c = 1; c <= 6; c++) {
+    const int t = (nb + c - 1) / c;
+    const double w = t * (c + 0.5);
+    if (w < cost) {
+      cost = w;
+      best = c;
+    }
+  }
+  return best;
+}
+
+hipError_t launch_alm_gemm(const double *lam, const double *G, const int4 *tiles, const XcdRuns &xr,
+                           const int64_t *off, int m0, int lmax, int RP, int ldg, int ncols, double *alm, int ldo,
+                           hipStream_t s)
+{
+  const int c = alm_col_blocks(ncols), nct = ((ncols + 15) / 16 + c - 1) / c;
+  int per_xcd = 0;
+  for (int x = 0; x < 8; x++) per_xcd = std::max(per_xcd, xr.start[x + 1] - xr.start[x]);
+  const dim3 g((unsigned)(8 * per_xcd * nct));
+  switch (c) {
+#define CRIME_ALM(CC)                                                                                              \
+  case CC:                                                                                                         \
+    hipLaunchKernelGGL(k_alm_gemm<CC>, g, dim3(256), 0, s, lam, G, tiles, nct, xr, off, m0, lmax, RP, ldg, ncols,  \
+                       alm, ldo);                                                                                  \
+    break;
+    CRIME_ALM(1) CRIME_ALM(2) CRIME_ALM(3) CRIME_ALM(4) CRIME_ALM(5) CRIME_ALM(6)
+#undef CRIME_ALM
+  default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
@@ -1088,6 +1254,22 @@ hipError_t launch_cls_sets(const double *alm, int lmax, int nsets, int mps, int 
 {
   const int nt = (mps + GT - 1) / GT;
   const int nl = lmax + 1;
+  if (mps > GT && mps <= 4 * GT) {
+    const int64_t nb = (int64_t)8 * nsets * (((nl + 15) / 16 + 7) / 8) * 16;
+    if (nb > 0x7fffffff) return hipErrorInvalidValue;
+    const dim3 g((unsigned)nb);
+    switch ((mps + 15) / 16) {
+#define CRIME_CLS(NN)                                                                                          \
+  case NN:                                                                                                     \
+    hipLaunchKernelGGL(k_cls_triangle<NN>, g, dim3(CLS_THREADS), 0, s, alm, lmax, mps, ldo, cls);              \
+    break;
+      CRIME_CLS(5) CRIME_CLS(6) CRIME_CLS(7) CRIME_CLS(8) CRIME_CLS(9) CRIME_CLS(10) CRIME_CLS(11) CRIME_CLS(12)
+      CRIME_CLS(13) CRIME_CLS(14) CRIME_CLS(15) CRIME_CLS(16)
+#undef CRIME_CLS
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   const int64_t ngroups = (int64_t)nsets * nt * (nt + 1) / 2;   // (set, tile pair) groups of nl blocks
   const int64_t nblk = ngroups * nl;
   if (nblk > 0x7fffffff) return hipErrorInvalidValue;
