@@ -1,7 +1,8 @@
 // Stockham autosort FFT engine for gfx950: one workgroup transforms a tile of lines of length L.
 //
-// Layout of the work: a line is split over TC threads; thread t owns E = L/TC elements, held in
-// VGPRs as B = E/R radix-R butterflies per pass (butterfly j = t + b*TC).  Pass p reads element
+// Layout of the work: a line is split over TC threads; in a radix-R pass thread t computes the butterflies
+// j = t + b*TC < L/R, b < B = ceil(L/R / TC), held in VGPRs (where TC does not divide L/R, as for the
+// 3*2^a lengths, some threads have one butterfly less in that pass).  Pass p reads element
 // j + s*L/R, applies the twiddles exp(+2 pi i s (j mod Ns)/(Ns R)) and a radix-R DFT, and writes
 // element (j/Ns)*Ns*R + (j mod Ns) + s*Ns (Stockham autosort, so no bit reversal is needed).
 // Pass 0 reads through a caller functor (global memory or an on-the-fly generator), intermediate
@@ -67,10 +68,14 @@ constexpr RadixPlan make_plan(int L, int maxr = 16)
 
 constexpr int cgcd(int a, int b) { return b == 0 ? a : cgcd(b, a % b); }
 
-// largest number of threads per line such that every pass has a whole number of butterflies per
-// thread, capped at tcmax
+// threads per line.  2^a lengths: the most that give every pass a whole number of butterflies per thread, capped
+// at tcmax.  3*2^a lengths: L/12, which leaves at most 16 elements per thread in every pass (one radix-16, two
+// radix-8, three radix-4 or four radix-3 butterflies).  Whole numbers of butterflies would allow them L/48 or so
+// threads with 48 elements each: the 192^3 FP32 passes
+// then took 116 + 26 + 43 us, now 55 + 23 + 33, and the fill of 48^3 94 us, now 12
 constexpr int plan_tc(int L, int tcmax, int maxr = 16)
 {
+  if (L % 3 == 0) return L / 12;
   RadixPlan p = make_plan(L, maxr);
   int g = L / p.r[0];
   for (int i = 1; i < p.n; i++) g = cgcd(g, L / p.r[i]);
@@ -194,10 +199,32 @@ template <typename T, int L, int TC, int MAXR = 16>
 struct Stockham {
   static constexpr RadixPlan plan = make_plan(L, MAXR);
   static constexpr int NP = plan.n;
-  static constexpr int E = L / TC;
 
   template <int P>
   static constexpr int radix() { return plan.r[P]; }
+  // butterflies of pass P: all of them, and at most per thread; RAGGED: not the same number for every thread
+  template <int P>
+  static constexpr int nbf() { return L / plan.r[P]; }
+  template <int P>
+  static constexpr int bft() { return (L / plan.r[P] + TC - 1) / TC; }
+  template <int P>
+  static constexpr bool ragged() { return (L / plan.r[P]) % TC != 0; }
+  static constexpr int emax()
+  {
+    int e = 0;
+    for (int i = 0; i < plan.n; i++) {
+      const int n = (L / plan.r[i] + TC - 1) / TC * plan.r[i];
+      if (n > e) e = n;
+    }
+    return e;
+  }
+  static constexpr int E = emax();   // elements per thread, at most
+  // barriers of run(): a workgroup's other waves take part in them through idle()
+  template <bool LoadFromLds = false>
+  __device__ static __forceinline__ void idle()
+  {
+    for (int i = 0; i < 2 * (NP - 1) + (LoadFromLds ? 1 : 0); i++) __syncthreads();
+  }
   template <int P>
   static constexpr int ns()
   {
@@ -221,9 +248,10 @@ struct Stockham {
   template <int P>
   __device__ static __forceinline__ void compute(cx<T> (&v)[E], int t, const cx<T> *__restrict__ tw)
   {
-    constexpr int R = radix<P>(), Ns = ns<P>(), B = E / R, TWS = L / (Ns * R);
+    constexpr int R = radix<P>(), Ns = ns<P>(), B = bft<P>(), TWS = L / (Ns * R);
 #pragma unroll
     for (int b = 0; b < B; ++b) {
+      if (ragged<P>() && t + b * TC >= nbf<P>()) continue;
       if constexpr (Ns > 1) {
         int k = (t + b * TC) % Ns;
 #pragma unroll
@@ -238,26 +266,32 @@ struct Stockham {
                                               const cx<T> *__restrict__ tw)
   {
     compute<P>(v, t, tw);
-    constexpr int R = radix<P>(), B = E / R;
+    constexpr int R = radix<P>(), B = bft<P>();
     if constexpr (P + 1 < NP) {
 #pragma unroll
-      for (int b = 0; b < B; ++b)
+      for (int b = 0; b < B; ++b) {
+        if (ragged<P>() && t + b * TC >= nbf<P>()) continue;
 #pragma unroll
         for (int s = 0; s < R; ++s) lds(out_index<P>(t, b, s)) = v[b * R + s];
+      }
       __syncthreads();
-      constexpr int R2 = radix<P + 1>(), B2 = E / R2;
+      constexpr int R2 = radix<P + 1>(), B2 = bft<P + 1>();
 #pragma unroll
-      for (int b = 0; b < B2; ++b)
+      for (int b = 0; b < B2; ++b) {
+        if (ragged<P + 1>() && t + b * TC >= nbf<P + 1>()) continue;
 #pragma unroll
         for (int s = 0; s < R2; ++s) v[b * R2 + s] = lds(in_index<P + 1>(t, b, s));
+      }
       __syncthreads();
       step<P + 1>(v, t, store, lds, tw);
     }
     else {
 #pragma unroll
-      for (int b = 0; b < B; ++b)
+      for (int b = 0; b < B; ++b) {
+        if (ragged<P>() && t + b * TC >= nbf<P>()) continue;
 #pragma unroll
         for (int s = 0; s < R; ++s) store(out_index<P>(t, b, s), v[b * R + s]);
+      }
     }
   }
 
@@ -268,11 +302,13 @@ struct Stockham {
                                              const cx<T> *__restrict__ tw)
   {
     cx<T> v[E];
-    constexpr int R = radix<0>(), B = E / R;
+    constexpr int R = radix<0>(), B = bft<0>();
 #pragma unroll
-    for (int b = 0; b < B; ++b)
+    for (int b = 0; b < B; ++b) {
+      if (ragged<0>() && t + b * TC >= nbf<0>()) continue;
 #pragma unroll
       for (int s = 0; s < R; ++s) v[b * R + s] = load(in_index<0>(t, b, s));
+    }
     if constexpr (LoadFromLds) __syncthreads();
     step<0>(v, t, store, lds, tw);
   }

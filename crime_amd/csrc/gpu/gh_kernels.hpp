@@ -39,7 +39,7 @@ constexpr int emax() { return sizeof(T) == 4 ? 64 : 32; }
 // 0 only for the FFT stages.
 constexpr int N_SCHED = 4;
 constexpr int N_SCHED_PIX = 4;
-constexpr int CRIME_GH_SCHED_VERSION = 4;  // bump when a variant's meaning changes (schedule cache keys)
+constexpr int CRIME_GH_SCHED_VERSION = 5;  // bump when a variant's meaning changes (schedule cache keys)
 constexpr int TUNE_MIN_N = 128;
 struct Schedule {
   int fill = 0, y = 0, x = 0, pix = 0;
@@ -72,15 +72,30 @@ struct ColCfg {
 };
 
 // the fused fill + kz pass only writes (64-byte write requests waste nothing): a tile of at most
-// 64 KB keeps two workgroups per CU, so one's mode generation overlaps the other's FFT; the
-// variants take 32 KB or 128 KB tiles instead
+// 64 KB keeps two or more workgroups per CU, so one's mode generation overlaps another's FFT; the
+// variants take other widths, and 32 KB or 128 KB tiles above 512^3.  Default against 16 columns: 256^3 FP32
+// 104 us against 128, FP64 205 against 282, 384^3 300 against 576 (with 8 threads per column)
 template <typename T, int N, int V = 0>
 struct FillCfg {
   static constexpr int MAXR = fft_maxr(V);
   static constexpr int W = fft_tiling(V);
   static constexpr int TC = ColCfg<T, N, V>::TC;
-  static constexpr int TX = cmin(ColCfg<T, N, V>::tx_for(W == 0 ? 65536 : (W == 1 ? 32768 : 131072)), 1024 / TC);
+  // columns: columns longer than 1 KB and up to 512^3 eight of them by default (variant 0) and sixteen in variant 1, shorter and
+  // longer ones the other way round
+  static constexpr bool NARROW = 8 * TC >= 64 && N * (int)sizeof(cx<T>) > 1024 && N <= 512;
+  static constexpr int TXT = W == 2 ? 4 : ((W == 0) == NARROW ? 8 : 16);
+  static constexpr int BUDGET = W == 2 ? 131072 : (W == 0 ? 65536 : 32768);
+  static constexpr int tx_for()
+  {
+    int tx = cmin(TXT, cpow2_div(N));
+    while (tx > 1 && tx * ColCfg<T, N, V>::CB > BUDGET) tx /= 2;
+    return tx;
+  }
+  static constexpr int TX = cmin(tx_for(), 1024 / TC);
   static constexpr int NT = TX * TC;
+  // threads per workgroup: small grids have few, so more waves draw the modes (a mode is a serial chain of a
+  // thousand instructions) and then sit out the transform
+  static constexpr int NTG = NT % 64 == 0 && NT < 256 ? 256 : NT;
 };
 
 // contiguous kx pass: TY rows per workgroup, TC threads per row; the variants take half or twice the
@@ -93,7 +108,8 @@ struct RowCfg {
   static constexpr int RB = N * (int)sizeof(cx<T>);
   static constexpr int ty_for(int budget)
   {
-    int ty = cmin(cmax(256 / TC, 1), cpow2_div(N * N));
+    // grids below 128 have fewer rows than would fill 256 CUs with 256-thread workgroups
+    int ty = cmin(cmax((N < 128 ? 64 : 256) / TC, 1), cpow2_div(N * N));
     while (ty > 1 && ty * RB > budget) ty /= 2;
     return ty;
   }

@@ -155,7 +155,7 @@ __device__ __forceinline__ cx<T> fill_element_a(const FillParams &f, cx<T> ab, i
 // kernels
 // ---------------------------------------------------------------------------------------------
 template <typename T, int N, int V>
-__global__ __launch_bounds__((FillCfg<T, N, V>::NT)) void k_fill_z(cx<T> *__restrict__ F, FillParams f,
+__global__ __launch_bounds__((FillCfg<T, N, V>::NTG)) void k_fill_z(cx<T> *__restrict__ F, FillParams f,
                                                                  const cx<T> *__restrict__ tw)
 {
   using C = FillCfg<T, N, V>;
@@ -173,12 +173,16 @@ __global__ __launch_bounds__((FillCfg<T, N, V>::NT)) void k_fill_z(cx<T> *__rest
   const AmpEntry<T> *amp = (const AmpEntry<T> *)f.amp;
   // kz = e and N - e in one step: one read of their shared amplitude (a scattered gather, a cache line per
   // lane) for two elements
-  for (int e = t; e <= N / 2; e += C::TC) {
+  for (int e = t; e <= N / 2; e += C::NTG / C::TX) {
     const cx<T> ab = mode_amp<T, N>(f, amp, kx, ky, e);
     lds[e * C::TX + c] = fill_element_a<T, N>(f, ab, kx, ky, e);
     if (e > 0 && e < N / 2) lds[(N - e) * C::TX + c] = fill_element_a<T, N>(f, ab, kx, ky, N - e);
   }
   __syncthreads();
+  if (C::NTG > C::NT && threadIdx.x >= C::NT) {   // whole waves
+    Stockham<T, N, C::TC, C::MAXR>::template idle<true>();
+    return;
+  }
   auto load = [&](int e) { return lds[e * C::TX + c]; };
   auto store = [&](int e, cx<T> v) { col[(size_t)e * n2] = v; };
   auto slot = [&](int e) -> cx<T> & { return lds[e * C::TX + c]; };
@@ -381,7 +385,7 @@ template <typename T, int N, int V>
 static void launch_fill_v(cx<T> *F, const FillParams &f, const cx<T> *tw, hipStream_t s)
 {
   using FC = FillCfg<T, N, V>;
-  hipLaunchKernelGGL((k_fill_z<T, N, V>), dim3(N / FC::TX, N), dim3(FC::NT), 0, s, F, f, tw);
+  hipLaunchKernelGGL((k_fill_z<T, N, V>), dim3(N / FC::TX, N), dim3(FC::NTG), 0, s, F, f, tw);
 }
 
 template <typename T, int N, int V>
