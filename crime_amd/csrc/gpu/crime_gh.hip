@@ -38,16 +38,18 @@ struct crime_gh {
   void *d_amp = nullptr;       // amplitude per |k|^2
   uint32_t *d_order = nullptr; // map-stage tiles by distance from the observer
   uint32_t *d_binstart = nullptr; // [nbins + 1] first tile of each distance bin in d_order
-  uint32_t *d_range = nullptr; // [2] the map kernel's range of d_order (k_tile_range)
-  uint8_t *d_cull = nullptr;   // [ntiles] out-of-band flags of d_order's entries (k_tile_cull)
+  uint32_t *d_range = nullptr; // [2] the map kernel's range of d_order (k_map_prep)
+  uint8_t *d_cull = nullptr;   // [ntiles] out-of-band flags of d_order's entries (k_map_prep)
   double *d_sub = nullptr;     // [3*n_sub]
   double *d_subp = nullptr;    // [3*n_sub] the offsets in the map stage's visiting order
   double *d_modes = nullptr;   // injected unit modes
   void *d_tw = nullptr;        // twiddles exp(+2 pi i m/N)
   double *d_partials = nullptr;
   double *d_sig = nullptr;     // [sigma2, mean, max |phi| of the grid (infinite when unknown)]
-  double *h_sig = nullptr;     // pinned mirror
-  uint32_t *h_range = nullptr; // pinned mirror of d_range (the map stage's grid)
+  unsigned long long *d_stamp = nullptr; // [N_STAMPS] stage times of the current run
+  double ms_per_tick = 0;      // of the stamps
+  RunEnd *h_end = nullptr, *h_end_dev = nullptr;   // pinned: what a run hands back (host and device address)
+  uint32_t *h_range = nullptr, *h_range_dev = nullptr; // pinned copy of d_range (the map stage's grid), likewise
   hipEvent_t ev_range = nullptr;
   int nparts = 0;
   FillParams fill{};
@@ -56,7 +58,7 @@ struct crime_gh {
   bool fields_done = false;
   double eps_nu = 0;           // frequency margin of the FP32 screen (MHz)
   Schedule sched{};            // kernel variants (crime_gh_autotune / crime_gh_set_schedule)
-  hipEvent_t ev[8] = {};
+  hipEvent_t ev[3] = {};       // of the point sources
   // point sources (allocated by the first crime_gh_mk_psources_maps)
   double *d_ps = nullptr;      // nz[PS_NZ] | maxpdf[PS_NZ] | c1[n_nu] | c2[n_nu] | A[npix] | B[npix]
   unsigned long long *d_ps_count = nullptr;
@@ -326,10 +328,10 @@ static void twiddles(int n, std::vector<cx<T>> &tw)
 static int free_all(crime_gh *h)
 {
   void *ptrs[] = {h->F, h->G, h->d_sin, h->d_fx, h->d_fxs, h->d_chwin, h->maps, h->d_tab, h->d_pk, h->d_edges, h->d_prefac, h->d_crec, h->d_amp, h->d_order, h->d_binstart, h->d_range, h->d_cull, h->d_sub, h->d_subp,
-                  h->d_modes, h->d_tw, h->d_partials, h->d_sig, h->d_ps, h->d_ps_count, h->ps_maps};
+                  h->d_modes, h->d_tw, h->d_partials, h->d_sig, h->d_stamp, h->d_ps, h->d_ps_count, h->ps_maps};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
-  if (h->h_sig) (void)hipHostFree(h->h_sig);
+  if (h->h_end) (void)hipHostFree(h->h_end);
   if (h->h_range) (void)hipHostFree(h->h_range);
   for (auto &e : h->ev)
     if (e) (void)hipEventDestroy(e);
@@ -396,6 +398,14 @@ static int create_impl(const crime_gh_desc *d, crime_gh *h)
   for (auto &e : h->ev) HIP_OR_FAIL(h, hipEventCreate(&e));
   HIP_OR_FAIL(h, hipEventCreateWithFlags(&h->ev_range, hipEventDisableTiming));
   HIP_OR_FAIL(h, hipHostMalloc((void **)&h->h_range, 2 * sizeof(uint32_t), hipHostMallocDefault));
+  HIP_OR_FAIL(h, hipHostGetDevicePointer((void **)&h->h_range_dev, h->h_range, 0));
+  HIP_OR_FAIL(h, hipHostMalloc((void **)&h->h_end, sizeof(RunEnd), hipHostMallocDefault));
+  HIP_OR_FAIL(h, hipHostGetDevicePointer((void **)&h->h_end_dev, h->h_end, 0));
+  HIP_OR_FAIL(h, hipMalloc((void **)&h->d_stamp, N_STAMPS * sizeof(unsigned long long)));
+  HIP_OR_FAIL(h, hipMemset(h->d_stamp, 0, N_STAMPS * sizeof(unsigned long long)));
+  int khz = 0;
+  HIP_OR_FAIL(h, hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, d->device));
+  h->ms_per_tick = khz > 0 ? 1.0 / khz : 0.0;
 
   HIP_OR_FAIL(h, hipMalloc(&h->F, h->ncell * 2 * esz));
   if (d->velocity_mode == CRIME_GH_VEL_SPECTRAL) {
@@ -424,9 +434,8 @@ static int create_impl(const crime_gh_desc *d, crime_gh *h)
   HIP_OR_FAIL(h, hipMalloc((void **)&h->d_subp, 3 * (size_t)d->n_sub * sizeof(double)));
   HIP_OR_FAIL(h, hipMalloc(&h->d_tw, h->n * 2 * esz));
   h->nparts = fields_partials_count(h->n, h->prec);
-  HIP_OR_FAIL(h, hipMalloc((void **)&h->d_partials, 3 * (size_t)h->nparts * sizeof(double)));
+  HIP_OR_FAIL(h, hipMalloc((void **)&h->d_partials, fields_partials_doubles(h->nparts) * sizeof(double)));
   HIP_OR_FAIL(h, hipMalloc((void **)&h->d_sig, 3 * sizeof(double)));
-  HIP_OR_FAIL(h, hipHostMalloc((void **)&h->h_sig, 2 * sizeof(double), hipHostMallocDefault));
   size_t nhalf = (size_t)h->n * h->n * (h->n / 2 + 1);
   if (d->mode_source == CRIME_GH_MODES_INJECTED) {
     HIP_OR_FAIL(h, hipMalloc((void **)&h->d_modes, 2 * nhalf * sizeof(double)));
@@ -722,12 +731,14 @@ static int enqueue_fields(crime_gh *h, bool timed, hipStream_t s = nullptr)
 {
   hipError_t e;
   if (!s) s = h->stream;
+  FillParams f = h->fill;
+  f.stamp = timed ? h->d_stamp : nullptr;
   if (h->prec)
-    e = launch_fields<double>(h->n, (cx<double> *)h->F, (cx<double> *)h->G, h->fill, (const cx<double> *)h->d_tw, h->norm,
-                              h->d_partials, h->d_sig, s, timed ? h->ev : nullptr, h->sched);
+    e = launch_fields<double>(h->n, (cx<double> *)h->F, (cx<double> *)h->G, f, (const cx<double> *)h->d_tw, h->norm,
+                              h->d_partials, h->d_sig, s, h->sched);
   else
-    e = launch_fields<float>(h->n, (cx<float> *)h->F, (cx<float> *)h->G, h->fill, (const cx<float> *)h->d_tw, h->norm,
-                             h->d_partials, h->d_sig, s, timed ? h->ev : nullptr, h->sched);
+    e = launch_fields<float>(h->n, (cx<float> *)h->F, (cx<float> *)h->G, f, (const cx<float> *)h->d_tw, h->norm,
+                             h->d_partials, h->d_sig, s, h->sched);
   if (e != hipSuccess) return set_error(h, CRIME_GH_EHIP, "field kernels: %s", hipGetErrorString(e));
   return 0;
 }
@@ -737,37 +748,51 @@ static int enqueue_fields(crime_gh *h, bool timed, hipStream_t s = nullptr)
 static int enqueue_maps(crime_gh *h, bool timed, hipStream_t s = nullptr)
 {
   hipError_t e;
-  const RangeReadback rb{h->h_range, h->ev_range};
+  const RangeReadback rb{h->h_range, h->h_range_dev, h->ev_range};
   const RangeReadback *prb = s ? nullptr : &rb;
   if (!s) s = h->stream;
+  MapParams m = h->map;
+  m.stamp = timed ? h->d_stamp : nullptr;
   if (h->prec)
-    e = launch_maps<double>((const cx<double> *)h->F, (double *)h->maps, h->nmaps, h->map, s,
-                            timed ? h->ev + 5 : nullptr, h->sched, prb);
+    e = launch_maps<double>((const cx<double> *)h->F, (double *)h->maps, h->nmaps, m, s, h->sched, prb);
   else
-    e = launch_maps<float>((const cx<float> *)h->F, (float *)h->maps, h->nmaps, h->map, s,
-                           timed ? h->ev + 5 : nullptr, h->sched, prb);
+    e = launch_maps<float>((const cx<float> *)h->F, (float *)h->maps, h->nmaps, m, s, h->sched, prb);
   if (e != hipSuccess) return set_error(h, CRIME_GH_EHIP, "map kernels: %s", hipGetErrorString(e));
+  return 0;
+}
+
+// time between two stamps of the run that h_end holds
+static double stamp_ms(const crime_gh *h, int a, int b)
+{
+  return (double)(int64_t)(h->h_end->stamp[b] - h->h_end->stamp[a]) * h->ms_per_tick;
+}
+
+// waits for the run; sigma^2 and the stamps then lie in h_end
+static int wait_run(crime_gh *h)
+{
+  HIP_OR_FAIL(h, launch_run_end(h->d_sig, h->d_stamp, h->h_end_dev, h->stream));
+  HIP_OR_FAIL(h, hipStreamSynchronize(h->stream));
   return 0;
 }
 
 static int finish(crime_gh *h, crime_gh_stats *st, bool fields, bool maps)
 {
-  HIP_OR_FAIL(h, hipMemcpyAsync(h->h_sig, h->d_sig, 2 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  HIP_OR_FAIL(h, hipStreamSynchronize(h->stream));
+  const int rc = wait_run(h);
+  if (rc) return rc;
   if (st) {
     if (fields) {
-      st->ms_fill_fft_z = ev_ms(h->ev[0], h->ev[1]);
-      st->ms_fft_y = ev_ms(h->ev[1], h->ev[2]);
-      st->ms_fft_x = ev_ms(h->ev[2], h->ev[3]);
-      st->ms_sigma2 = ev_ms(h->ev[3], h->ev[4]);
+      st->ms_fill_fft_z = stamp_ms(h, STAMP_FILL, STAMP_Y);
+      st->ms_fft_y = stamp_ms(h, STAMP_Y, STAMP_X);
+      st->ms_fft_x = stamp_ms(h, STAMP_X, STAMP_SIGMA);
+      st->ms_sigma2 = stamp_ms(h, STAMP_SIGMA, STAMP_FIELDS_END);
     }
     if (maps) {
-      st->ms_maps_clear = ev_ms(h->ev[5], h->ev[6]);
-      st->ms_pixelize = ev_ms(h->ev[6], h->ev[7]);
+      st->ms_maps_clear = stamp_ms(h, STAMP_MAPS, STAMP_SCATTER);
+      st->ms_pixelize = stamp_ms(h, STAMP_SCATTER, STAMP_END);
     }
-    st->ms_total = ev_ms(fields ? h->ev[0] : h->ev[5], maps ? h->ev[7] : h->ev[4]);
-    st->sigma2_gauss = h->h_sig[0];
-    st->mean_gauss = h->h_sig[1];
+    st->ms_total = stamp_ms(h, fields ? STAMP_FILL : STAMP_MAPS, maps ? STAMP_END : STAMP_FIELDS_END);
+    st->sigma2_gauss = h->h_end->sig[0];
+    st->mean_gauss = h->h_end->sig[1];
   }
   return 0;
 }
@@ -968,8 +993,9 @@ extern "C" int crime_gh_autotune(crime_gh_t *h, int reps, int *sched_out, double
       for (int r = 0; r < reps; r++) {
         int rc = enqueue_fields(h, true);
         if (rc) return rc;
-        HIP_OR_FAIL(h, hipStreamSynchronize(h->stream));
-        double ms = ev_ms(h->ev[stage], h->ev[stage + 1]);
+        rc = wait_run(h);
+        if (rc) return rc;
+        const double ms = stamp_ms(h, STAMP_FILL + stage, STAMP_FILL + stage + 1);
         if (ms >= 0 && ms < t) t = ms;
       }
       table[stage][v] = t;
@@ -989,8 +1015,9 @@ extern "C" int crime_gh_autotune(crime_gh_t *h, int reps, int *sched_out, double
     for (int r = 0; r < reps; r++) {
       rc = enqueue_maps(h, true);
       if (rc) return rc;
-      HIP_OR_FAIL(h, hipStreamSynchronize(h->stream));
-      double ms = ev_ms(h->ev[6], h->ev[7]);
+      rc = wait_run(h);
+      if (rc) return rc;
+      const double ms = stamp_ms(h, STAMP_SCATTER, STAMP_END);
       if (ms >= 0 && ms < t) t = ms;
     }
     table[3][v] = t;

@@ -119,6 +119,14 @@ struct RowCfg {
   static constexpr int NT = TY * TC;
 };
 
+// Times of a run's stages: the device's wall clock (hipDeviceAttributeWallClockRate) as the first workgroup of a
+// stage's first kernel starts.  An event between two kernels would hold the second back by about 5 us.
+enum { STAMP_FILL, STAMP_Y, STAMP_X, STAMP_SIGMA, STAMP_FIELDS_END, STAMP_MAPS, STAMP_SCATTER, STAMP_END, N_STAMPS };
+__device__ __forceinline__ void stamp(unsigned long long *st, int i)
+{
+  if (st && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) st[i] = wall_clock64();
+}
+
 struct FillParams {
   int n;
   double dk, idk3, f0h0, r2_smooth;
@@ -137,6 +145,7 @@ struct FillParams {
   // v_j(k) = i sin_dx[m_j] phi_k and sin_dx[m] = sin(2 pi m / N) / dx (exactly 0 at m = 0, N/2)
   int vmode, comp;
   const double *sin_dx;
+  unsigned long long *stamp;  // [N_STAMPS] or NULL
 };
 
 // amplitude-table entry: A (FP32 grids) or (A, A psi) (FP64 grids)
@@ -197,7 +206,7 @@ struct MapParams {
   int nbins;
   double tile_hd;              // every cell centre of a tile lies within tile_hd of the tile's centre
   uint32_t *tile_range;        // device [first, last): the entries of tile_order the map kernel visits
-  uint8_t *tile_cull;          // device [ntiles]: 1 when tile_order's entry i is out of the band (k_tile_cull;
+  uint8_t *tile_cull;          // device [ntiles]: 1 when tile_order's entry i is out of the band (k_map_prep;
                                // written for the range only)
   int ntx, nty, ntz;
   int vmode;               // CRIME_GH_VEL_*: SPECTRAL reads vx from F.y and (vy, vz) from G
@@ -208,6 +217,7 @@ struct MapParams {
   unsigned long long *fxmaps;
   double *fxs;
   double *mass_part;
+  unsigned long long *stamp;   // [N_STAMPS] or NULL
   ScreenParams scr;
 };
 
@@ -249,24 +259,36 @@ hipError_t launch_ps_expand(const double *A, const double *B, const double *c1, 
 // sigma^2 partials are those of F, whose kx pass runs last).
 template <typename T>
 hipError_t launch_fields(int n, cx<T> *F, cx<T> *G, const FillParams &f, const cx<T> *tw, double norm,
-                         double *partials, double *sig, hipStream_t s, hipEvent_t *ev, const Schedule &sc);
+                         double *partials, double *sig, hipStream_t s, const Schedule &sc);
 
 constexpr int PK_MAX_BINS = 2048;
 template <typename T>
 hipError_t launch_power_spectrum(int n, cx<T> *F, const cx<T> *tw, double pscale, double binw, int nbins,
                                  double *acc, hipStream_t s);
-int fields_partials_count(int n, int prec);
+int fields_partials_count(int n, int prec);   // row blocks of the kx pass, at most
+constexpr int SIGMA_BLOCKS = 256;             // blocks of the first step of a long sigma^2 reduction
+// doubles of the sigma^2 partials: three per row block and per block of the first step
+inline size_t fields_partials_doubles(int nparts) { return 3 * ((size_t)nparts + SIGMA_BLOCKS); }
 
 // The map stage's tile range to the host: with it, launch_maps waits (on the host, while the maps are
-// cleared) for the range k_tile_range found and launches exactly its workgroups; without it (a stream under
-// capture) the launch covers every tile and the workgroups past the range exit on their first load.
+// cleared) for the range k_map_prep found and launches exactly its workgroups; without it (a stream under
+// capture) the launch covers every tile and the workgroups past the range exit on their first load, as they do
+// for up to RANGE_MIN_TILES tiles: an exit costs 1.6 ns, the wait about 20 us.
 struct RangeReadback {
-  uint32_t *h_range;   // pinned [2]
-  hipEvent_t ev;       // recorded after the copy of the range
+  uint32_t *h_range;   // pinned [2], as the host sees it
+  uint32_t *d_range;   // and as the device does
+  hipEvent_t ev;       // recorded after the range is written
 };
+constexpr size_t RANGE_MIN_TILES = 12000;
 template <typename T>
 hipError_t launch_maps(const cx<T> *F, T *maps, size_t nmaps, const MapParams &m, hipStream_t s,
-                       hipEvent_t *ev, const Schedule &sc, const RangeReadback *rb = nullptr);
+                       const Schedule &sc, const RangeReadback *rb = nullptr);
+// the end of a run: sigma^2, <delta> and the stamps to pinned host memory
+struct RunEnd {
+  double sig[2];
+  unsigned long long stamp[N_STAMPS];
+};
+hipError_t launch_run_end(const double *sig, unsigned long long *stamps, RunEnd *out, hipStream_t s);
 template <typename T>
 hipError_t launch_cell_field(const cx<T> *F, const MapParams &m, int which, size_t cell0, size_t ncell, double *out,
                              hipStream_t s);

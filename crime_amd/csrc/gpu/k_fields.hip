@@ -160,6 +160,7 @@ __global__ __launch_bounds__((FillCfg<T, N, V>::NTG)) void k_fill_z(cx<T> *__res
 {
   using C = FillCfg<T, N, V>;
   __shared__ cx<T> lds[N * C::TX];
+  stamp(f.stamp, STAMP_FILL);
   const int c = threadIdx.x % C::TX, t = threadIdx.x / C::TX;
   // Blocks go to the XCDs round-robin (XCD = linear block index mod 8), and N / TX is a multiple of 8,
   // so without a rotation every row's kx = 0 and kx = N/2 blocks -- whose waves run the one-draw and the
@@ -191,10 +192,11 @@ __global__ __launch_bounds__((FillCfg<T, N, V>::NTG)) void k_fill_z(cx<T> *__res
 
 template <typename T, int N, int V>
 __global__ __launch_bounds__((ColCfg<T, N, V>::NT)) void k_fft_y(cx<T> *__restrict__ F,
-                                                               const cx<T> *__restrict__ tw)
+                                                               const cx<T> *__restrict__ tw, unsigned long long *st)
 {
   using C = ColCfg<T, N, V>;
   __shared__ cx<T> lds[N * C::TX];
+  stamp(st, STAMP_Y);
   const int c = threadIdx.x % C::TX, t = threadIdx.x / C::TX;
   // XCD-aware tile order: neighbouring column tiles of one plane run on one XCD, so tiles narrower
   // than a 128-byte line share each line through that XCD's L2 instead of fetching it twice
@@ -211,9 +213,10 @@ template <typename T, int N, int V>
 __global__ __launch_bounds__((RowCfg<T, N, V>::NT)) void k_fft_x(cx<T> *__restrict__ F,
                                                                const cx<T> *__restrict__ tw,
                                                                double norm, double norm_phi,
-                                                               double *__restrict__ partials)
+                                                               double *__restrict__ partials, unsigned long long *st)
 {
   using C = RowCfg<T, N, V>;
+  stamp(st, STAMP_X);
   __shared__ cx<T> lds[N * C::TY];
   __shared__ double red[2 * C::NT];
   __shared__ unsigned long long imax;
@@ -323,7 +326,7 @@ static hipError_t launch_pk_n(cx<T> *F, const cx<T> *tw, double pscale, double b
   using CC = ColCfg<T, N>;
   using RC = RowCfg<T, N>;
   hipLaunchKernelGGL((k_fft_x_conj<T, N>), dim3((N * N) / RC::TY), dim3(RC::NT), 0, s, F, tw);
-  hipLaunchKernelGGL((k_fft_y<T, N, 0>), dim3(N / CC::TX, N), dim3(CC::NT), 0, s, F, tw);
+  hipLaunchKernelGGL((k_fft_y<T, N, 0>), dim3(N / CC::TX, N), dim3(CC::NT), 0, s, F, tw, (unsigned long long *)nullptr);
   hipLaunchKernelGGL((k_fft_z<T, N>), dim3(N / CC::TX, N), dim3(CC::NT), 0, s, F, tw);
   size_t n3 = (size_t)N * N * N;
   unsigned nb = (unsigned)((n3 + 255) / 256 < 8192 ? (n3 + 255) / 256 : 8192);
@@ -348,34 +351,80 @@ template hipError_t launch_power_spectrum<float>(int, cx<float> *, const cx<floa
 template hipError_t launch_power_spectrum<double>(int, cx<double> *, const cx<double> *, double, double, int,
                                                   double *, hipStream_t);
 
-__global__ __launch_bounds__(1024) void k_sigma_finalize(const double *__restrict__ partials, int nparts,
-                                                         double ncells, double *__restrict__ out)
+// Partials of n blocks: sums p[2 i], sums of squares p[2 i + 1], largest |imaginary part| p[2 n + i].  The block's
+// thread t takes the entries of index t mod NT (from first, every stride), then a tree: a fixed order.
+template <int NT>
+__device__ __forceinline__ void sigma_reduce(const double *__restrict__ p, int n, int first, int stride, double &a,
+                                             double &b, double &c)
 {
-  __shared__ double r1[1024], r2[1024], r3[1024];
-  double a = 0, b = 0, c = 0;
-  for (int i = threadIdx.x; i < nparts; i += 1024) {
-    a += partials[2 * i];
-    b += partials[2 * i + 1];
-    c = fmax(c, partials[2 * nparts + i]);
+  __shared__ double r1[NT], r2[NT], r3[NT];
+  a = b = c = 0;
+  for (int i = first; i < n; i += stride) {
+    a += p[2 * i];
+    b += p[2 * i + 1];
+    c = fmax(c, p[2 * n + i]);
   }
-  r1[threadIdx.x] = a;
-  r2[threadIdx.x] = b;
-  r3[threadIdx.x] = c;
+  const int t = threadIdx.x;
+  r1[t] = a;
+  r2[t] = b;
+  r3[t] = c;
   __syncthreads();
-  for (int w = 512; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      r1[threadIdx.x] += r1[threadIdx.x + w];
-      r2[threadIdx.x] += r2[threadIdx.x + w];
-      r3[threadIdx.x] = fmax(r3[threadIdx.x], r3[threadIdx.x + w]);
+  for (int w = NT / 2; w > 0; w >>= 1) {
+    if (t < w) {
+      r1[t] += r1[t + w];
+      r2[t] += r2[t + w];
+      r3[t] = fmax(r3[t], r3[t + w]);
     }
     __syncthreads();
   }
+  a = r1[0];
+  b = r2[0];
+  c = r3[0];
+}
+
+// first step of a long reduction: one workgroup over 1024^3's half million partials took 265 us
+__global__ __launch_bounds__(256) void k_sigma_blocks(const double *__restrict__ p, int n, double *__restrict__ out,
+                                                      unsigned long long *st)
+{
+  stamp(st, STAMP_SIGMA);
+  double a, b, c;
+  sigma_reduce<256>(p, n, blockIdx.x * 256 + threadIdx.x, 256 * SIGMA_BLOCKS, a, b, c);
   if (threadIdx.x == 0) {
-    double mean = r1[0] / ncells;
-    out[0] = r2[0] / ncells - mean * mean;  // sigma2_gauss (fourier.c:74)
-    out[1] = mean;
-    out[2] = r3[0];  // max |imaginary part| of the grid (the map stage's bound on the velocity)
+    out[2 * blockIdx.x] = a;
+    out[2 * blockIdx.x + 1] = b;
+    out[2 * SIGMA_BLOCKS + blockIdx.x] = c;
   }
+}
+
+__global__ __launch_bounds__(1024) void k_sigma_finalize(const double *__restrict__ partials, int nparts, double ncells,
+                                                         double *__restrict__ out, unsigned long long *st,
+                                                         unsigned long long *st_end)
+{
+  stamp(st, STAMP_SIGMA);
+  double a, b, c;
+  sigma_reduce<1024>(partials, nparts, threadIdx.x, 1024, a, b, c);
+  if (threadIdx.x == 0) {
+    double mean = a / ncells;
+    out[0] = b / ncells - mean * mean;  // sigma2_gauss (fourier.c:74)
+    out[1] = mean;
+    out[2] = c;  // max |imaginary part| of the grid (the map stage's bound on the velocity)
+    stamp(st_end, STAMP_FIELDS_END);
+  }
+}
+
+__global__ __launch_bounds__(64) void k_run_end(const double *__restrict__ sig, unsigned long long *stamps,
+                                                RunEnd *__restrict__ out)
+{
+  const int t = threadIdx.x;
+  if (t < 2) out->sig[t] = sig[t];
+  if (t < N_STAMPS) out->stamp[t] = t == STAMP_END ? (unsigned long long)wall_clock64() : stamps[t];
+  __threadfence_system();
+}
+
+hipError_t launch_run_end(const double *sig, unsigned long long *stamps, RunEnd *out, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_run_end, dim3(1), dim3(64), 0, s, sig, stamps, out);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -389,18 +438,19 @@ static void launch_fill_v(cx<T> *F, const FillParams &f, const cx<T> *tw, hipStr
 }
 
 template <typename T, int N, int V>
-static void launch_y_v(cx<T> *F, const cx<T> *tw, hipStream_t s)
+static void launch_y_v(cx<T> *F, const cx<T> *tw, hipStream_t s, unsigned long long *st)
 {
   using CC = ColCfg<T, N, V>;
-  hipLaunchKernelGGL((k_fft_y<T, N, V>), dim3(N / CC::TX, N), dim3(CC::NT), 0, s, F, tw);
+  hipLaunchKernelGGL((k_fft_y<T, N, V>), dim3(N / CC::TX, N), dim3(CC::NT), 0, s, F, tw, st);
 }
 
 template <typename T, int N, int V>
-static int launch_x_v(cx<T> *F, const cx<T> *tw, double norm, double norm_phi, double *partials, hipStream_t s)
+static int launch_x_v(cx<T> *F, const cx<T> *tw, double norm, double norm_phi, double *partials, hipStream_t s,
+                      unsigned long long *st)
 {
   using RC = RowCfg<T, N, V>;
   const int nrowblk = (N * N) / RC::TY;
-  hipLaunchKernelGGL((k_fft_x<T, N, V>), dim3(nrowblk), dim3(RC::NT), 0, s, F, tw, norm, norm_phi, partials);
+  hipLaunchKernelGGL((k_fft_x<T, N, V>), dim3(nrowblk), dim3(RC::NT), 0, s, F, tw, norm, norm_phi, partials, st);
   return nrowblk;
 }
 
@@ -415,61 +465,64 @@ static void fill_sched(cx<T> *F, const FillParams &f, const cx<T> *tw, hipStream
 }
 
 template <typename T, int N>
-static void y_sched(cx<T> *F, const cx<T> *tw, hipStream_t s, const Schedule &sc)
+static void y_sched(cx<T> *F, const cx<T> *tw, hipStream_t s, const Schedule &sc, unsigned long long *st)
 {
   constexpr bool tuned = N >= TUNE_MIN_N;
-  if (tuned && sc.y == 1) launch_y_v<T, N, tuned ? 1 : 0>(F, tw, s);
-  else if (tuned && sc.y == 2) launch_y_v<T, N, tuned ? 2 : 0>(F, tw, s);
-  else if (tuned && sc.y == 3) launch_y_v<T, N, tuned ? 3 : 0>(F, tw, s);
-  else launch_y_v<T, N, 0>(F, tw, s);
+  if (tuned && sc.y == 1) launch_y_v<T, N, tuned ? 1 : 0>(F, tw, s, st);
+  else if (tuned && sc.y == 2) launch_y_v<T, N, tuned ? 2 : 0>(F, tw, s, st);
+  else if (tuned && sc.y == 3) launch_y_v<T, N, tuned ? 3 : 0>(F, tw, s, st);
+  else launch_y_v<T, N, 0>(F, tw, s, st);
 }
 
 template <typename T, int N>
 static int x_sched(cx<T> *F, const cx<T> *tw, double nre, double nim, double *partials, hipStream_t s,
-                   const Schedule &sc)
+                   const Schedule &sc, unsigned long long *st)
 {
   constexpr bool tuned = N >= TUNE_MIN_N;
-  if (tuned && sc.x == 1) return launch_x_v<T, N, tuned ? 1 : 0>(F, tw, nre, nim, partials, s);
-  if (tuned && sc.x == 2) return launch_x_v<T, N, tuned ? 2 : 0>(F, tw, nre, nim, partials, s);
-  if (tuned && sc.x == 3) return launch_x_v<T, N, tuned ? 3 : 0>(F, tw, nre, nim, partials, s);
-  return launch_x_v<T, N, 0>(F, tw, nre, nim, partials, s);
+  if (tuned && sc.x == 1) return launch_x_v<T, N, tuned ? 1 : 0>(F, tw, nre, nim, partials, s, st);
+  if (tuned && sc.x == 2) return launch_x_v<T, N, tuned ? 2 : 0>(F, tw, nre, nim, partials, s, st);
+  if (tuned && sc.x == 3) return launch_x_v<T, N, tuned ? 3 : 0>(F, tw, nre, nim, partials, s, st);
+  return launch_x_v<T, N, 0>(F, tw, nre, nim, partials, s, st);
 }
 
-// Stage timings (ev[0..4]) cover both grids of a spectral handle: the second grid's pass runs right
-// before the same pass of F, and its sigma^2 partials are overwritten by F's kx pass.
+// Stage times cover both grids of a spectral handle: the second grid's pass runs right before the same pass of F
+// (and is the one stamped), and its sigma^2 partials are overwritten by F's kx pass.
 template <typename T, int N>
 static hipError_t launch_fields_n(cx<T> *F, cx<T> *G, const FillParams &f, const cx<T> *tw, double norm,
-                                  double *partials, double *sig, hipStream_t s, hipEvent_t *ev,
-                                  const Schedule &sc)
+                                  double *partials, double *sig, hipStream_t s, const Schedule &sc)
 {
   const bool two = f.vmode != 0;
-  FillParams f1 = f;
+  unsigned long long *const st = f.stamp, *const st2 = two ? nullptr : st;
+  FillParams f0 = f, f1 = f;
+  f0.stamp = st2;
   f1.comp = 1;
-  if (ev) (void)hipEventRecord(ev[0], s);
   if (two) fill_sched<T, N>(G, f1, tw, s, sc);
-  fill_sched<T, N>(F, f, tw, s, sc);
-  if (ev) (void)hipEventRecord(ev[1], s);
-  if (two) y_sched<T, N>(G, tw, s, sc);
-  y_sched<T, N>(F, tw, s, sc);
-  if (ev) (void)hipEventRecord(ev[2], s);
+  fill_sched<T, N>(F, f0, tw, s, sc);
+  if (two) y_sched<T, N>(G, tw, s, sc, st);
+  y_sched<T, N>(F, tw, s, sc, st2);
   const double nphi = norm / f.phi_scale;
-  if (two) x_sched<T, N>(G, tw, nphi, nphi, partials, s, sc);
-  const int nrowblk = x_sched<T, N>(F, tw, norm, nphi, partials, s, sc);
-  if (ev) (void)hipEventRecord(ev[3], s);
-  hipLaunchKernelGGL(k_sigma_finalize, dim3(1), dim3(1024), 0, s, partials, nrowblk,
-                     (double)N * N * N, sig);
-  if (ev) (void)hipEventRecord(ev[4], s);
+  if (two) x_sched<T, N>(G, tw, nphi, nphi, partials, s, sc, st);
+  int n = x_sched<T, N>(F, tw, norm, nphi, partials, s, sc, st2);
+  unsigned long long *sts = st;
+  if (n > 16 * SIGMA_BLOCKS) {
+    double *out = partials + 3 * (size_t)n;
+    hipLaunchKernelGGL(k_sigma_blocks, dim3(SIGMA_BLOCKS), dim3(256), 0, s, partials, n, out, st);
+    partials = out;
+    n = SIGMA_BLOCKS;
+    sts = nullptr;
+  }
+  hipLaunchKernelGGL(k_sigma_finalize, dim3(1), dim3(1024), 0, s, partials, n, (double)N * N * N, sig, sts, st);
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_fields(int n, cx<T> *F, cx<T> *G, const FillParams &f, const cx<T> *tw, double norm,
-                         double *partials, double *sig, hipStream_t s, hipEvent_t *ev, const Schedule &sc)
+                         double *partials, double *sig, hipStream_t s, const Schedule &sc)
 {
   if (f.vmode != 0 && (!G || !f.sin_dx)) return hipErrorInvalidValue;
   switch (n) {
 #define CRIME_CASE(NN) \
-  case NN: return launch_fields_n<T, NN>(F, G, f, tw, norm, partials, sig, s, ev, sc);
+  case NN: return launch_fields_n<T, NN>(F, G, f, tw, norm, partials, sig, s, sc);
     CRIME_FOR_EACH_N(CRIME_CASE)
 #undef CRIME_CASE
   default: return hipErrorInvalidValue;
@@ -477,9 +530,9 @@ hipError_t launch_fields(int n, cx<T> *F, cx<T> *G, const FillParams &f, const c
 }
 
 template hipError_t launch_fields<float>(int, cx<float> *, cx<float> *, const FillParams &, const cx<float> *,
-                                         double, double *, double *, hipStream_t, hipEvent_t *, const Schedule &);
+                                         double, double *, double *, hipStream_t, const Schedule &);
 template hipError_t launch_fields<double>(int, cx<double> *, cx<double> *, const FillParams &, const cx<double> *,
-                                          double, double *, double *, hipStream_t, hipEvent_t *, const Schedule &);
+                                          double, double *, double *, hipStream_t, const Schedule &);
 
 template <typename T>
 hipError_t launch_amp_table(const FillParams &f, void *tab, hipStream_t s)

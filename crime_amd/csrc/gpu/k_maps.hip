@@ -611,6 +611,7 @@ __device__ __forceinline__ void pixelize_body(const cx<T> *__restrict__ F, T *__
   __shared__ K keys[SLOTS];
   __shared__ V vals[SLOTS];
   __shared__ DeferQueue dq;
+  stamp(m.stamp, STAMP_SCATTER);
   V *__restrict__ vmaps;
   if constexpr (FX) vmaps = m.fxmaps;
   else vmaps = maps;
@@ -619,12 +620,12 @@ __device__ __forceinline__ void pixelize_body(const cx<T> *__restrict__ F, T *__
   // tiles run in order of distance from the observer, so the workgroups resident at one time cover a
   // thin shell and their atomics fall on a few channels of the maps.  2-D grid: a dispatch holds at
   // most 2^32 work-items per dimension.
-  // the workgroups take the entries [first, last) of the order that k_tile_range kept; the rest exit here
+  // the workgroups take the entries [first, last) of the order that k_map_prep kept; the rest exit here
   const size_t bid = (size_t)m.tile_range[0] + (size_t)blockIdx.y * gridDim.x + blockIdx.x;
   if (bid >= (size_t)m.tile_range[1]) return;
   const uint32_t b = m.tile_order[bid];
   const int tx = (int)(b & 1023u), ty = (int)((b >> 10) & 1023u), tz = (int)(b >> 20);
-  // whole tiles out of the band, by the grid's bound on the RSD shift (k_tile_cull): before any grid load
+  // whole tiles out of the band, by the grid's bound on the RSD shift (k_map_prep): before any grid load
   if (m.tile_cull[bid]) return;
   const int ix = tx * TILE_X + (t % TILE_X), iy = ty * TILE_Y + ((t / TILE_X) % TILE_Y),
             iz = tz * TILE_Z + t / (TILE_X * TILE_Y);
@@ -749,41 +750,69 @@ __device__ __forceinline__ void pixelize_body(const cx<T> *__restrict__ F, T *__
   }
 }
 
-// The range [first, last) of tile_order that the map kernel visits, for the current grid's RSD bound: from
-// the first entry of the nearest distance bin that bin_out_of_band keeps to the last entry of the farthest
-// (every tile when the bound is off).  One workgroup, before the map kernel.
-__global__ __launch_bounds__(256) void k_tile_range(MapParams m)
+// The map kernel's preparation, by block: 0 the range [first, last) of tile_order that it visits, for the current
+// grid's RSD bound, from the first entry of the nearest distance bin that bin_out_of_band keeps to the last entry of
+// the farthest (every tile when the bound is off), also to h_range if given; up to tile_blocks the out-of-band flag
+// of every entry of tile_order, one tile per thread, which the map kernel's workgroups read instead of each
+// evaluating the test; the others clear CLEAR_BYTES each of the accumulated maps.
+constexpr size_t CLEAR_BYTES = 16384;
+__device__ __forceinline__ void clear_block(uint4 *p, size_t nbytes, size_t block)
+{
+  const size_t nv = nbytes / 16, first = block * (CLEAR_BYTES / 16) + threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < (int)(CLEAR_BYTES / 4096); i++) {
+    const size_t j = first + 256 * i;
+    if (j < nv) p[j] = make_uint4(0, 0, 0, 0);
+  }
+  // the last words, fewer than 16 bytes of them
+  if (block == 0 && threadIdx.x < (nbytes % 16) / 4) ((uint32_t *)(p + nv))[threadIdx.x] = 0;
+}
+
+__global__ __launch_bounds__(256) void k_clear(uint4 *p, size_t nbytes) { clear_block(p, nbytes, blockIdx.x); }
+
+__global__ __launch_bounds__(256) void k_map_prep(MapParams m, unsigned tile_blocks, uint32_t *h_range, uint4 *clr,
+                                                  size_t nbytes)
 {
   __shared__ int lo, hi;
-  if (threadIdx.x == 0) {
-    lo = 0x7fffffff;
-    hi = -1;
-  }
-  __syncthreads();
+  stamp(m.stamp, STAMP_MAPS);
   const double dzb = m.precull ? m.dz_per_phi * m.sig[2] : INFINITY;
-  for (int b = threadIdx.x; b < m.nbins; b += 256)
-    if (m.bin_start[b] < m.bin_start[b + 1] && !bin_out_of_band(m, b, dzb)) {
-      atomicMin(&lo, b);
-      atomicMax(&hi, b);
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) {
+      lo = 0x7fffffff;
+      hi = -1;
     }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const bool any = lo <= hi;
-    m.tile_range[0] = any ? m.bin_start[lo] : 0u;
-    m.tile_range[1] = any ? m.bin_start[hi + 1] : 0u;
+    __syncthreads();
+    for (int b = threadIdx.x; b < m.nbins; b += 256)
+      if (m.bin_start[b] < m.bin_start[b + 1] && !bin_out_of_band(m, b, dzb)) {
+        atomicMin(&lo, b);
+        atomicMax(&hi, b);
+      }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const bool any = lo <= hi;
+      const uint32_t r0 = any ? m.bin_start[lo] : 0u, r1 = any ? m.bin_start[hi + 1] : 0u;
+      m.tile_range[0] = r0;
+      m.tile_range[1] = r1;
+      if (h_range) {
+        h_range[0] = r0;
+        h_range[1] = r1;
+        __threadfence_system();
+      }
+    }
+  }
+  else if (blockIdx.x < tile_blocks) {
+    const size_t i = (size_t)(blockIdx.x - 1) * 256 + threadIdx.x;
+    if (i >= (size_t)m.ntx * m.nty * m.ntz) return;
+    const uint32_t b = m.tile_order[i];
+    const int tx = (int)(b & 1023u), ty = (int)((b >> 10) & 1023u), tz = (int)(b >> 20);
+    m.tile_cull[i] = m.precull && tile_out_of_band(m, tx, ty, tz, dzb) ? 1 : 0;
+  }
+  else {
+    clear_block(clr, nbytes, blockIdx.x - tile_blocks);
   }
 }
 
-// The out-of-band flag of every entry of tile_order in [first, last), one tile per thread, with the grid's RSD
-// bound (0 when the bound is off): the map kernel's workgroups read it instead of each evaluating the test.
-__global__ __launch_bounds__(256) void k_tile_cull(MapParams m)
-{
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < (size_t)m.tile_range[0] || i >= (size_t)m.tile_range[1]) return;
-  const uint32_t b = m.tile_order[i];
-  const int tx = (int)(b & 1023u), ty = (int)((b >> 10) & 1023u), tz = (int)(b >> 20);
-  m.tile_cull[i] = m.precull && tile_out_of_band(m, tx, ty, tz, m.dz_per_phi * m.sig[2]) ? 1 : 0;
-}
+__global__ void k_stamp(unsigned long long *st, int i) { stamp(st, i); }
 
 template <typename T, int SLOTS, int SEG, bool FX, typename K>
 __global__ __launch_bounds__(256) void k_pixelize(const cx<T> *__restrict__ F, T *__restrict__ maps, MapParams m)
@@ -806,6 +835,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_mass_partials(const cx<T> *__restrict__ F, MapParams m)
 {
   __shared__ double red[256];
+  stamp(m.stamp, STAMP_SCATTER);
   const size_t ncell = (size_t)m.n * m.n * m.n;
   double acc = 0;
   for (size_t cell = (size_t)blockIdx.x * 256 + threadIdx.x; cell < ncell; cell += (size_t)FX_PARTS * 256) {
@@ -1451,57 +1481,50 @@ static void launch_pixelize(const cx<T> *F, T *maps, const MapParams &m, hipStre
   else run(I2048{}, S2{}, true);
 }
 
-// ev[0] before clearing, ev[1] before the scatter, ev[2] after the last map kernel
 template <typename T>
-hipError_t launch_maps(const cx<T> *F, T *maps, size_t nmaps, const MapParams &m, hipStream_t s,
-                       hipEvent_t *ev, const Schedule &sc, const RangeReadback *rb)
+hipError_t launch_maps(const cx<T> *F, T *maps, size_t nmaps, const MapParams &m, hipStream_t s, const Schedule &sc,
+                       const RangeReadback *rb)
 {
-  if (ev) (void)hipEventRecord(ev[0], s);
-  hipLaunchKernelGGL(k_tile_range, dim3(1), dim3(256), 0, s, m);
-  {
-    const size_t nt = (size_t)m.ntx * m.nty * m.ntz;
-    hipLaunchKernelGGL(k_tile_cull, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, m);
-  }
+  if (m.fx && (!m.fxmaps || !m.fxs || !m.mass_part)) return hipErrorInvalidValue;
+  const size_t ntiles = (size_t)m.ntx * m.nty * m.ntz;
+  if (ntiles <= RANGE_MIN_TILES) rb = nullptr;
+  const unsigned tile_blocks = 1 + (unsigned)((ntiles + 255) / 256);
+  uint4 *clr = m.fx ? (uint4 *)m.fxmaps : (uint4 *)maps;
+  const size_t nbytes = nmaps * (m.fx ? sizeof(unsigned long long) : sizeof(T));
+  const unsigned clear_blocks = (unsigned)((nbytes + CLEAR_BYTES - 1) / CLEAR_BYTES);
+  size_t launch = ntiles;   // the workgroups: the range's size when the host has it, else every tile
   if (rb) {
-    hipError_t e = hipMemcpyAsync(rb->h_range, m.tile_range, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipEventRecord(rb->ev, s);
+    // the range alone first: the clear runs while the host waits for it
+    hipLaunchKernelGGL(k_map_prep, dim3(tile_blocks), dim3(256), 0, s, m, tile_blocks, rb->d_range, clr, nbytes);
+    hipError_t e = hipEventRecord(rb->ev, s);
     if (e != hipSuccess) return e;
-  }
-  if (m.fx) {
-    if (!m.fxmaps || !m.fxs || !m.mass_part) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_zero<unsigned long long>, dim3(nblk(nmaps)), dim3(256), 0, s, m.fxmaps, nmaps);
+    hipLaunchKernelGGL(k_clear, dim3(clear_blocks), dim3(256), 0, s, clr, nbytes);
   }
   else {
-    hipLaunchKernelGGL(k_zero<T>, dim3(nblk(nmaps)), dim3(256), 0, s, maps, nmaps);
+    hipLaunchKernelGGL(k_map_prep, dim3(tile_blocks + clear_blocks), dim3(256), 0, s, m, tile_blocks,
+                       (uint32_t *)nullptr, clr, nbytes);
   }
-  if (ev) (void)hipEventRecord(ev[1], s);
-  // the workgroups: the range's size when the host has it (the clear above runs meanwhile), else every tile
-  size_t ntiles = (size_t)m.ntx * m.nty * m.ntz;
-  auto host_range = [&]() -> hipError_t {
-    const hipError_t e = hipEventSynchronize(rb->ev);
-    if (e == hipSuccess) ntiles = rb->h_range[1] > rb->h_range[0] ? rb->h_range[1] - rb->h_range[0] : 0;
-    return e;
-  };
+  MapParams mp = m;
   if (m.fx) {
     hipLaunchKernelGGL(k_mass_partials<T>, dim3(FX_PARTS), dim3(256), 0, s, F, m);
     hipLaunchKernelGGL(k_fx_scale, dim3(1), dim3(256), 0, s, m);
-    if (rb) {
-      const hipError_t e = host_range();
-      if (e != hipSuccess) return e;
-    }
-    launch_pixelize<T, true>(F, maps, m, s, sc, ntiles);
+    mp.stamp = nullptr;   // the scatter's time starts with the mass
+  }
+  if (rb) {
+    const hipError_t e = hipEventSynchronize(rb->ev);
+    if (e != hipSuccess) return e;
+    launch = rb->h_range[1] > rb->h_range[0] ? rb->h_range[1] - rb->h_range[0] : 0;
+  }
+  if (launch == 0 && mp.stamp) hipLaunchKernelGGL(k_stamp, dim3(1), dim3(64), 0, s, mp.stamp, (int)STAMP_SCATTER);
+  if (m.fx) {
+    launch_pixelize<T, true>(F, maps, mp, s, sc, launch);
     int64_t b = (m.npix + 255) / 256;
     hipLaunchKernelGGL(k_fx_finalize<T>, dim3((unsigned)(b < 4096 ? b : 4096), m.n_nu), dim3(256), 0, s,
                        (const unsigned long long *)m.fxmaps, maps, m);
   }
   else {
-    if (rb) {
-      const hipError_t e = host_range();
-      if (e != hipSuccess) return e;
-    }
-    launch_pixelize<T, false>(F, maps, m, s, sc, ntiles);
+    launch_pixelize<T, false>(F, maps, mp, s, sc, launch);
   }
-  if (ev) (void)hipEventRecord(ev[2], s);
   return hipGetLastError();
 }
 
@@ -1588,7 +1611,7 @@ hipError_t launch_ps_expand(const double *A, const double *B, const double *c1, 
 
 #define CRIME_INST(T)                                                                                   \
   template hipError_t launch_maps<T>(const cx<T> *, T *, size_t, const MapParams &, hipStream_t,      \
-                                     hipEvent_t *, const Schedule &, const RangeReadback *);            \
+                                     const Schedule &, const RangeReadback *);                          \
   template hipError_t launch_cell_field<T>(const cx<T> *, const MapParams &, int, size_t, size_t, double *,   \
                                            hipStream_t);                                                \
   template hipError_t launch_sample_indices<T>(const cx<T> *, const MapParams &, int64_t, int64_t,     \

@@ -117,7 +117,7 @@ typedef struct crime_gh_desc {
   int32_t deterministic;      /* 1: bit-reproducible maps (fixed-point scatter, see below) (ABI 2) */
 } crime_gh_desc;
 
-/* per-call timings (hipEvent, ms) and diagnostics */
+/* per-call timings (ms, from the device's clock at the start of each stage) and diagnostics */
 typedef struct crime_gh_stats {
   double ms_fill_fft_z;       /* mode fill fused with the kz pass */
   double ms_fft_y;
