@@ -8,7 +8,12 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+#include <condition_variable>
+#include <exception>
+#include <mutex>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -132,7 +137,10 @@ struct RowArgs {
   size_t stride;                 // elements per layer of hp, dzp
   int n, npart;                  // rows; partials allocated per layer in part_b
   int gather;
+  float scale;                   // forward: not 0: write scale sinh(y) (the emulator's spectra) for y
 };
+
+__device__ __forceinline__ float spectrum(float y, float scale) { return (float)sinh((double)y) * scale; }
 
 // One workgroup takes BM rows through the whole network without leaving the CU: the activations of the
 // current layer stay in one LDS tile, the weights stream from L2 as fragments (prefetched across the
@@ -294,7 +302,7 @@ __global__ __launch_bounds__(row_threads(NT), 4) void k_mlp_rows(RowArgs g)
   }
   __syncthreads();
   if constexpr (!TRAIN) {
-    if (tid < BM && row0 + tid < g.n) g.Y[row0 + tid] = ds[tid];
+    if (tid < BM && row0 + tid < g.n) g.Y[row0 + tid] = g.scale != 0.0f ? spectrum(ds[tid], g.scale) : ds[tid];
     return;
   }
   else {
@@ -557,6 +565,12 @@ struct crime_mlp {
   hipGraphExec_t exec = nullptr;
   int graph_batch = 0;
   int use_graph = 1;                        // 0: every step enqueued directly (crime_mlp_set_graph)
+  // crime_mlp_predict: pinned inputs and outputs of `slots` chunks of `slot_rows` rows, and the inputs' device copies
+  // (more than one slot), sent on a stream of their own
+  int slots = 0, slot_rows = 0;
+  float *hx = nullptr, *hy = nullptr, *hx_dev = nullptr, *hy_dev = nullptr, *dx = nullptr;
+  std::vector<hipEvent_t> slot_in, slot_ev;   // a slot's inputs are on the device; its outputs in hy
+  hipStream_t copy = nullptr;
   std::string err;
 };
 
@@ -596,12 +610,28 @@ static void drop_graph(crime_mlp *h)
   h->graph_batch = 0;
 }
 
+static void drop_slots(crime_mlp *h)
+{
+  if (h->hx) (void)hipHostFree(h->hx);
+  if (h->hy) (void)hipHostFree(h->hy);
+  if (h->dx) (void)hipFree(h->dx);
+  for (hipEvent_t e : h->slot_in) (void)hipEventDestroy(e);
+  for (hipEvent_t e : h->slot_ev) (void)hipEventDestroy(e);
+  h->hx = h->hy = h->hx_dev = h->hy_dev = h->dx = nullptr;
+  h->slot_in.clear();
+  h->slot_ev.clear();
+  h->slots = h->slot_rows = 0;
+}
+
 extern "C" void crime_mlp_destroy(crime_mlp_t *h)
 {
   if (!h) return;
   (void)hipSetDevice(h->device);
   if (h->stream) (void)hipStreamSynchronize(h->stream);
+  if (h->copy) (void)hipStreamSynchronize(h->copy);
   drop_graph(h);
+  drop_slots(h);
+  if (h->copy) (void)hipStreamDestroy(h->copy);
   void *bufs[] = {h->p, h->m, h->v, h->grad, h->wf, h->wb, h->X, h->T, h->Wt, h->Y, h->hp, h->dzp,
                   h->part_in, h->part_out, h->part_b, h->st, h->loss, h->Xall, h->Tall, h->Wall};
   for (void *b : bufs)
@@ -611,6 +641,31 @@ extern "C" void crime_mlp_destroy(crime_mlp_t *h)
 }
 
 static int nred_of(int n) { return (n + RROWS - 1) / RROWS; }
+
+constexpr int PRED_DIRECT = 4096;   // rows of a call that needs no copies (crime_mlp_predict)
+static int ensure_slots(crime_mlp *h, int slots, int rows)
+{
+  if (slots <= h->slots && rows <= h->slot_rows) return 0;
+  slots = std::max(slots, h->slots);
+  rows = std::max(rows, h->slot_rows);
+  drop_slots(h);
+  const size_t n = (size_t)slots * rows;
+  MLP_HIP(h, hipHostMalloc((void **)&h->hx, n * NIN * sizeof(float), hipHostMallocDefault));
+  MLP_HIP(h, hipHostMalloc((void **)&h->hy, n * sizeof(float), hipHostMallocDefault));
+  MLP_HIP(h, hipHostGetDevicePointer((void **)&h->hx_dev, h->hx, 0));
+  MLP_HIP(h, hipHostGetDevicePointer((void **)&h->hy_dev, h->hy, 0));
+  if (slots > 1) {
+    MLP_HIP(h, hipMalloc((void **)&h->dx, n * NIN * sizeof(float)));
+    if (!h->copy) MLP_HIP(h, hipStreamCreateWithFlags(&h->copy, hipStreamNonBlocking));
+    h->slot_in.resize(slots, nullptr);
+    h->slot_ev.resize(slots, nullptr);
+    for (hipEvent_t &e : h->slot_in) MLP_HIP(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    for (hipEvent_t &e : h->slot_ev) MLP_HIP(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  h->slots = slots;
+  h->slot_rows = rows;
+  return 0;
+}
 
 static int create_impl(crime_mlp *h, int max_batch, int device)
 {
@@ -647,7 +702,7 @@ static int create_impl(crime_mlp *h, int max_batch, int device)
   MLP_HIP(h, hipMemcpy(h->p, zero.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice));
   MLP_HIP(h, hipMemcpy(h->m, zero.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice));
   MLP_HIP(h, hipMemcpy(h->v, zero.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice));
-  return 0;
+  return ensure_slots(h, 1, std::min(PRED_DIRECT, max_batch));   // a first short call finds them
 }
 
 extern "C" int crime_mlp_create(int max_batch, int device, crime_mlp_t **out)
@@ -718,11 +773,14 @@ static RowArgs row_args(crime_mlp *h, int n)
 // forward for rows [0, n) of X (the handle's own input buffer unless given) on stream s (its own unless given).
 // The fewest rows per workgroup that still give every one of the 256 CUs at most one workgroup, as the layers'
 // latency counts there (256 rows: 13 us by 16, 20 us by 32); above that 64 rows, which read the weights less often.
-static void enqueue_forward(crime_mlp *h, int n, hipStream_t s = nullptr, const float *X = nullptr)
+static void enqueue_forward(crime_mlp *h, int n, hipStream_t s = nullptr, const float *X = nullptr, float *Y = nullptr,
+                            float scale = 0.0f)
 {
   if (!s) s = h->stream;
   RowArgs g = row_args(h, n);
   if (X) g.X = X;
+  if (Y) g.Y = Y;
+  g.scale = scale;
   auto launch = [&](auto bm, auto nt) {
     constexpr int BM = decltype(bm)::value, NT = decltype(nt)::value;
     hipLaunchKernelGGL((k_mlp_rows<BM, NT, false>), dim3((n + BM - 1) / BM), dim3(row_threads(NT)), 0, s, g);
@@ -834,6 +892,196 @@ extern "C" int crime_mlp_forward_mean(crime_mlp_t *const *hs, int nh, int64_t n,
   }
   MLP_HIP(h0, hipStreamSynchronize(s));
   return 0;
+}
+
+__global__ __launch_bounds__(256) void k_spectra(const float *__restrict__ y, int n, float scale, float *__restrict__ out)
+{
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = spectrum(y[i], scale);
+}
+
+// rows [r0, r1) of the raw inputs as the network takes them: FP32, column 6 as (nu' - nu) / channel width
+static void encode_rows(const double *x, int64_t r0, int64_t r1, float inv_dnu, float *out)
+{
+  for (int64_t r = r0; r < r1; r++, out += NIN) {
+    for (int i = 0; i < NIN; i++) out[i] = (float)x[r * NIN + i];
+    out[6] = (out[6] - out[5]) * inv_dnu;
+  }
+}
+
+// Threads that encode the chunks of a call into the ring of slots, ENC_ROWS rows at a time in order; a chunk waits
+// until its slot was given back.  Joined when it goes out of scope, however the call ends.
+struct Encoders {
+  static constexpr int ENC_ROWS = 4096;
+  const double *x;
+  int64_t n;
+  int rows, slots;          // per chunk; ring
+  float inv_dnu;
+  float *hx;
+  std::mutex mu;
+  std::condition_variable cv;
+  std::vector<int> left;    // blocks of each chunk not yet encoded
+  int64_t next = 0;         // block to take
+  int64_t open;             // chunks that may be written: [0, open)
+  bool stop = false;
+  std::vector<std::thread> workers;
+
+  Encoders(const double *x_, int64_t n_, int rows_, int slots_, float inv_dnu_, float *hx_)
+      : x(x_), n(n_), rows(rows_), slots(slots_), inv_dnu(inv_dnu_), hx(hx_), open(slots_)
+  {
+    for (int64_t c0 = 0; c0 < n; c0 += rows) left.push_back((int)((std::min(n - c0, (int64_t)rows) + ENC_ROWS - 1) / ENC_ROWS));
+  }
+  // encodes blocks; main: until chunk `until` is complete, else until none is left
+  void work(int64_t until)
+  {
+    const int bpc = (rows + ENC_ROWS - 1) / ENC_ROWS;
+    std::unique_lock<std::mutex> lk(mu);
+    while (!stop) {
+      if (until >= 0 && left[until] == 0) return;
+      const int64_t c = next / bpc;
+      if (c >= (int64_t)left.size() || c >= open) {
+        if (until < 0 && c >= (int64_t)left.size()) return;
+        cv.wait(lk);
+        continue;
+      }
+      const int64_t b = next++ % bpc, r0 = c * rows + b * ENC_ROWS;
+      const int64_t r1 = std::min(n, std::min(r0 + ENC_ROWS, (c + 1) * (int64_t)rows));
+      if (r0 >= r1) continue;   // the last chunk has fewer blocks
+      lk.unlock();
+      encode_rows(x, r0, r1, inv_dnu, hx + ((size_t)(c % slots) * rows + (size_t)b * ENC_ROWS) * NIN);
+      lk.lock();
+      if (--left[c] == 0) cv.notify_all();
+    }
+  }
+  void start(int count)
+  {
+    for (int i = 0; i < count; i++) {
+      try {
+        workers.emplace_back([this] { work(-1); });
+      }
+      catch (const std::exception &) {
+        return;   // fewer threads: the caller encodes too
+      }
+    }
+  }
+  void give_back(int64_t chunk)
+  {
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      open = chunk + 1 + slots;
+    }
+    cv.notify_all();
+  }
+  ~Encoders()
+  {
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      stop = true;
+    }
+    cv.notify_all();
+    for (std::thread &t : workers) t.join();
+  }
+};
+
+// A call of up to PRED_DIRECT rows: the kernel reads the pinned inputs and writes the pinned outputs itself, no
+// copies between (256 rows: 28 us, against 42 with the two copies).  Longer ones run in chunks of PRED_ROWS: threads
+// encode (one thread would take as long as all the rest), a second stream sends a chunk's inputs while the networks
+// run on the one before, and outputs go straight to pinned memory and are handed out meanwhile.  A million rows:
+// 1.5 ms, of which 1.3 are the kernels', against 7.7 with the encoding, copies and sinh of the whole call one
+// after the other; chunks of 32768 rows with both copies on one stream 3.1, of 65536 2.5.
+constexpr int PRED_ROWS = 65536, PRED_SLOTS = 4, PRED_THREADS = 8;
+
+static int predict_impl(crime_mlp *const *hs, int nh, int64_t n, const double *x, float inv_dnu, float scale, float *y)
+{
+  crime_mlp *h = hs[0];
+  int batch = PRED_ROWS;
+  for (int k = 0; k < nh; k++) batch = std::min(batch, hs[k]->max_batch);
+  MLP_HIP(h, hipSetDevice(h->device));
+  for (int k = 1; k < nh; k++) MLP_HIP(h, hipStreamSynchronize(hs[k]->stream));  // no pending work on its buffers
+  const bool direct = n <= std::min(PRED_DIRECT, batch);
+  const int rows = direct ? (int)((n + 63) / 64 * 64) : batch;
+  const int64_t nchunks = (n + rows - 1) / rows;
+  int rc = ensure_slots(h, direct ? 1 : (int)std::max<int64_t>(2, std::min<int64_t>(PRED_SLOTS, nchunks)), rows);
+  if (rc) return rc;
+  hipStream_t s = h->stream;
+  // the networks on c rows of X, their spectra into Y
+  auto forward = [&](int c, const float *X, float *Y) {
+    if (nh == 1) {
+      enqueue_forward(h, c, s, X, Y, scale);
+      return;
+    }
+    for (int k = 0; k < nh; k++) {
+      enqueue_forward(hs[k], c, s, X);
+      hipLaunchKernelGGL(k_acc_rows, dim3((c + 255) / 256), dim3(256), 0, s, h->T, hs[k]->Y, c, 1.0f / (float)nh, k == 0);
+    }
+    hipLaunchKernelGGL(k_spectra, dim3((c + 255) / 256), dim3(256), 0, s, h->T, c, scale, Y);
+  };
+  if (direct) {
+    encode_rows(x, 0, n, inv_dnu, h->hx);
+    forward((int)n, h->hx_dev, h->hy_dev);
+    MLP_HIP(h, hipGetLastError());
+    MLP_HIP(h, hipStreamSynchronize(s));
+    memcpy(y, h->hy, (size_t)n * sizeof(float));
+    return 0;
+  }
+  const int slots = h->slots;
+  auto count = [&](int64_t c) { return (int)std::min<int64_t>(rows, n - c * rows); };
+  auto hand_out = [&](int64_t c) -> int {
+    MLP_HIP(h, hipEventSynchronize(h->slot_ev[c % slots]));
+    memcpy(y + c * rows, h->hy + (size_t)(c % slots) * rows, (size_t)count(c) * sizeof(float));
+    return 0;
+  };
+  Encoders enc(x, n, rows, slots, inv_dnu, h->hx);
+  enc.start((int)std::min<int64_t>(PRED_THREADS, n / (2 * Encoders::ENC_ROWS)));
+  int64_t out = 0;   // chunks handed out
+  for (int64_t c = 0; c < nchunks && !rc; c++) {
+    if (c - out >= slots - 1 && c > 0) {   // the oldest slot will be needed next
+      rc = hand_out(out);
+      enc.give_back(out++);
+      if (rc) break;
+    }
+    enc.work(c);
+    const size_t at = (size_t)(c % slots) * rows;
+    const int m = count(c);
+    // the slot's device inputs were read by a chunk that is handed out
+    MLP_HIP(h, hipMemcpyAsync(h->dx + at * NIN, h->hx + at * NIN, (size_t)m * NIN * sizeof(float), hipMemcpyHostToDevice,
+                              h->copy));
+    MLP_HIP(h, hipEventRecord(h->slot_in[c % slots], h->copy));
+    MLP_HIP(h, hipStreamWaitEvent(s, h->slot_in[c % slots], 0));
+    forward(m, h->dx + at * NIN, h->hy_dev + at);
+    MLP_HIP(h, hipGetLastError());
+    MLP_HIP(h, hipEventRecord(h->slot_ev[c % slots], s));
+  }
+  for (; out < nchunks && !rc; out++) rc = hand_out(out);
+  return rc;
+}
+
+static void drain(crime_mlp *h)
+{
+  if (h->copy) (void)hipStreamSynchronize(h->copy);
+  (void)hipStreamSynchronize(h->stream);
+}
+
+extern "C" int crime_mlp_predict(crime_mlp_t *const *hs, int nh, int64_t n, const double *x, float inv_dnu, float scale,
+                                 float *y)
+{
+  if (!hs || nh < 1 || !hs[0]) return mlp_error(nullptr, CRIME_GH_EINVAL, "need nh >= 1 handles");
+  crime_mlp *h = hs[0];
+  if (n < 1 || !x || !y || !(scale > 0)) return mlp_error(h, CRIME_GH_EINVAL, "need n >= 1, non-NULL x, y and scale > 0");
+  for (int k = 0; k < nh; k++) {
+    if (!hs[k]) return mlp_error(h, CRIME_GH_EINVAL, "handle %d is NULL", k);
+    if (hs[k]->device != h->device) return mlp_error(h, CRIME_GH_EINVAL, "handle %d is on another device", k);
+  }
+  try {
+    const int rc = predict_impl(hs, nh, n, x, inv_dnu, scale, y);
+    // nothing of a failed call may still read or write the slots
+    if (rc) drain(h);
+    return rc;
+  }
+  catch (const std::exception &e) {
+    drain(h);
+    return mlp_error(h, CRIME_GH_ENOMEM, "predict: %s", e.what());
+  }
 }
 
 extern "C" int crime_mlp_loss_grad(crime_mlp_t *h, int n, const float *x, const float *t, const float *w,

@@ -264,6 +264,17 @@ class Emulator:
 
     def predict(self, x):
         """Binned C_l at raw inputs x (n, 8).  Calls on one Emulator must not overlap (a shared input buffer)."""
+        x = np.asarray(x)
+        if (x.dtype == np.float64 and x.flags.c_contiguous and x.size >= NIN and x.size % NIN == 0
+                and np.float32(self.scale) > 0):
+            # encoding, networks and sinh in one call of the library (crime_mlp_predict)
+            n = x.size // NIN
+            y = np.empty(n, np.float32)
+            hs = (C.c_void_p * len(self.mlps))(*[m._h.value for m in self.mlps])
+            self.mlp._check(self.mlp._lib.crime_mlp_predict(
+                hs, len(self.mlps), n, x.ctypes.data_as(_ffi._dp), np.float32(1.0 / self.dnu), np.float32(self.scale),
+                _fp(y)))
+            return y
         y = self.predict_y(x)
         np.sinh(y, out=y)
         y *= np.float32(self.scale)

@@ -53,6 +53,11 @@ int crime_mlp_forward(crime_mlp_t *h, int64_t n, const float *x, float *y);
  * handles' own streams are synchronised first.  No counterpart in the reference (the emulator's). */
 int crime_mlp_forward_mean(crime_mlp_t *const *hs, int nh, int64_t n, const float *x, float *y);
 
+/* The emulator's spectra scale sinh(y) at raw FP64 inputs x[i][8] (Omega_m, sigma_8, n_s, h, b, nu, nu', log10 l):
+ * the networks' mean y at the inputs in FP32 with column 6 as (nu' - nu) inv_dnu.  Calls of one first handle must
+ * not overlap.  No counterpart in the reference (the emulator's). */
+int crime_mlp_predict(crime_mlp_t *const *hs, int nh, int64_t n, const double *x, float inv_dnu, float scale, float *y);
+
 /* Loss and its gradient (FP32, parameter order above) for one host batch, n <= max_batch, n % 64 == 0;
  * w may be NULL (unit weights).  The parameters are not changed. */
 int crime_mlp_loss_grad(crime_mlp_t *h, int n, const float *x, const float *t, const float *w, double *loss,
