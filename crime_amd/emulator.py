@@ -265,7 +265,7 @@ class Emulator:
     def predict(self, x):
         """Binned C_l at raw inputs x (n, 8).  Calls on one Emulator must not overlap (a shared input buffer)."""
         x = np.asarray(x)
-        if (x.dtype == np.float64 and x.flags.c_contiguous and x.size >= NIN and x.size % NIN == 0
+        if (x.dtype == np.float64 and x.flags.c_contiguous and x.flags.aligned and x.size >= NIN and x.size % NIN == 0
                 and np.float32(self.scale) > 0):
             # encoding, networks and sinh in one call of the library (crime_mlp_predict)
             n = x.size // NIN
