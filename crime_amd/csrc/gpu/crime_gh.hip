@@ -267,6 +267,32 @@ static int screen_setup(crime_gh *h, const crime_gh_desc *d, const std::vector<d
   return 0;
 }
 
+// Estimate of the bins that the samples of one tile occupy in the middle of the band: the tile spans
+// prod (length / bin size + 1) bins, for bins of the pixels' size there and the channels' mean depth, averaged
+// over the three axes as line of sight; of these S samples find all but exp(-S / bins).
+static double tile_bins(const MapParams &m, const crime_gh_desc *d, int64_t npix)
+{
+  auto r_of = [&](double z) {
+    int i = 0;
+    while (i + 1 < CRIME_GH_NZ && d->z_r2z[i + 1] < z) i++;
+    return d->r_r2z[i];
+  };
+  double far2 = 0;
+  for (int i = 0; i < 3; i++) {
+    const double f = fmax(fabs(m.obs[i]), fabs(d->l_box - m.obs[i]));
+    far2 += f * f;
+  }
+  const double rlo = r_of(CRIME_GH_NU_21 / m.nu_hi - 1);
+  const double rhi = m.nu_lo > 0 ? r_of(CRIME_GH_NU_21 / m.nu_lo - 1) : sqrt(far2);
+  const double depth = (rhi - rlo) / m.n_nu, pix = 0.5 * (rlo + fmin(rhi, sqrt(far2))) * sqrt(4 * M_PI / npix);
+  if (!(depth > 0) || !(pix > 0)) return 0;
+  const double len[3] = {TILE_X * m.dx, TILE_Y * m.dx, TILE_Z * m.dx};
+  double bins = 0;
+  for (int a = 0; a < 3; a++)
+    bins += (len[a] / depth + 1) * (len[(a + 1) % 3] / pix + 1) * (len[(a + 2) % 3] / pix + 1) / 3;
+  return bins * (1 - exp(-(double)TILE_X * TILE_Y * TILE_Z * m.n_sub / bins));
+}
+
 static int validate(const crime_gh_desc *d)
 {
   if (!d) return set_error(nullptr, CRIME_GH_EINVAL, "descriptor is NULL");
@@ -636,6 +662,8 @@ static int create_impl(const crime_gh_desc *d, crime_gh *h)
   m.n_guess = n_guess;
   m.g_lo = g_lo;
   m.g_inv = g_inv;
+
+  m.tile_bins = tile_bins(m, d, h->npix);
 
   // tile order for the map stage: counting sort of the tiles by the distance of their centre from
   // the observer, in bins of one cell

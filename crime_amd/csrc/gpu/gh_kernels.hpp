@@ -34,12 +34,13 @@ constexpr int emax() { return sizeof(T) == 4 ? 64 : 32; }
 
 // Schedule variants the autotuner chooses between, per stage (variant 0 is the default).  FFT stages:
 // variants 0-2 differ in tiling with radix-16 plans, variant 3 is variant 0's tiling with radix-8 plans
-// (one pass more, smaller butterflies).  Map stage: 2048 LDS bins grouped by 4 adjacent map words
-// (variant 0) or by 8 (variant 1), 4096 bins (2) and 1024 bins (3).  Grids below TUNE_MIN_N have variant
+// (one pass more, smaller butterflies).  Map stage: LDS bins grouped by 8 adjacent map words, 2048 or 4096 as the
+// estimate of a tile's bins says (variant 0), 2048 (1) or 4096 (2; 2048 with 64-bit keys), and 1024 grouped by 4 (3).
+// Grids below TUNE_MIN_N have variant
 // 0 only for the FFT stages.
 constexpr int N_SCHED = 4;
 constexpr int N_SCHED_PIX = 4;
-constexpr int CRIME_GH_SCHED_VERSION = 5;  // bump when a variant's meaning changes (schedule cache keys)
+constexpr int CRIME_GH_SCHED_VERSION = 7;  // bump when a variant's meaning changes (schedule cache keys)
 constexpr int TUNE_MIN_N = 128;
 struct Schedule {
   int fill = 0, y = 0, x = 0, pix = 0;
@@ -209,6 +210,7 @@ struct MapParams {
   uint8_t *tile_cull;          // device [ntiles]: 1 when tile_order's entry i is out of the band (k_map_prep;
                                // written for the range only)
   int ntx, nty, ntz;
+  double tile_bins;        // estimate of the (channel, pixel) bins that a tile's samples occupy
   int vmode;               // CRIME_GH_VEL_*: SPECTRAL reads vx from F.y and (vy, vz) from G
   const void *G;           // cx<T>[N^3] second grid of SPECTRAL handles (NULL otherwise)
   // deterministic scatter: integer mass sums in fx[n_nu * npix], scale s and 1/s in fxs[0..1],

@@ -487,8 +487,6 @@ __device__ __forceinline__ int sample_decide(const MapParams &m, const CellState
   return sample_bin(m, s, isub, ipix, pf);
 }
 
-// Add val to bin `key` of the workgroup's LDS table (open addressing, linear probing from slot h); a sample
-// that finds no slot within the probe budget goes straight to the map in HBM.
 template <typename T>
 __device__ __forceinline__ void global_add(T *p, T v)
 {
@@ -496,37 +494,46 @@ __device__ __forceinline__ void global_add(T *p, T v)
   else unsafeAtomicAdd(p, v);
 }
 
-// Home slot of a bin: the 2^SEG keys of one aligned run of map addresses (one 2^SEG-word segment) start at
-// a slot given by 32-bit Fibonacci hashing of the segment and follow each other from there, so that the
-// flush, where the lanes of a wave read consecutive slots, hands the lanes of one segment to one atomic
+// The slots of a bin: the 2^SEG keys of one aligned run of map addresses (one 2^SEG-word segment) share a
+// block of 2^SEG slots, given by 32-bit Fibonacci hashing of the segment, a key's place in it being its
+// place in the segment; a key whose place is taken tries the same place of the next blocks.  The flush,
+// where the lanes of a wave read consecutive slots, then hands the lanes of one segment to one atomic
 // instruction: the memory system merges the lanes of an instruction that fall into one segment (runs of
-// 4 lanes per 32-byte segment cost a third of scattered lanes).
+// 4 lanes per 32-byte segment cost a third of scattered lanes).  Runs that start at any slot and step by
+// one pile up behind each other: at 384^3 with 64 samples a cell a third of the kernel went into probes.
 template <int SLOTS, int SEG, typename K>
 __device__ __forceinline__ unsigned home_slot(K key)
 {
-  constexpr int SHIFT = 32 - __builtin_ctz(SLOTS);
+  constexpr int SHIFT = 32 - __builtin_ctz(SLOTS) + SEG;
   const K seg = key >> SEG;
   unsigned folded;
   if constexpr (sizeof(K) == 8) folded = (unsigned)seg ^ (unsigned)((unsigned long long)seg >> 32);
   else folded = (unsigned)seg;
-  return (((folded * 0x9E3779B1u) >> SHIFT) + ((unsigned)key & ((1u << SEG) - 1))) & (SLOTS - 1);
+  return (((folded * 0x9E3779B1u) >> SHIFT) << SEG) | ((unsigned)key & ((1u << SEG) - 1));
 }
 
-template <typename T, int SLOTS, typename K>
+// Slots that a sum tries before it goes to the map itself.  A wave probes as long as its unluckiest lane, and
+// in a full table every new bin tries them all.  Map stage at 4 / 8 / 16 / 64 probes: 384^3, Nside 256, 64 samples
+// a cell 7.3 / 7.5 / 7.9 / 9.1 ms; the same at Nside 512 (more bins than slots) 33 / 34 / 35 / 50 ms; 3 is level.
+constexpr int AGG_PROBES = 4;
+
+// Add val to bin `key` of the workgroup's LDS table, from slot h; a sum that finds no slot within the probe
+// budget goes straight to the map in HBM.
+template <typename T, int SLOTS, int SEG, typename K>
 __device__ __forceinline__ void agg_add(K key, unsigned h, T val, K *keys, T *vals, T *__restrict__ maps,
-                                        int probes = 64)
+                                        int probes = AGG_PROBES)
 {
   const K EMPTY = (K)~(K)0;
   // the compare-and-swap claims an empty slot and returns the key of an occupied one: one LDS round trip
-  // per probe (unrolled by 8 only: a collision is rare, and a longer chain costs scalar registers)
-#pragma unroll 8
+  // per probe
+#pragma unroll
   for (int p = 0; p < probes; p++) {
     const K old = atomicCAS(&keys[h], EMPTY, key);
     if (old == EMPTY || old == key) {
       atomicAdd(&vals[h], val);
       return;
     }
-    h = (h + 1) & (SLOTS - 1);
+    h = (h + (1u << SEG)) & (SLOTS - 1);
   }
   global_add(maps + key, val);
 }
@@ -542,7 +549,7 @@ struct PendingAdd {
   bool on;
 };
 
-template <typename T, int SLOTS, typename K>
+template <typename T, int SLOTS, int SEG, typename K>
 __device__ __forceinline__ void agg_start(PendingAdd<K, T> &pa, K key, unsigned h, T val, K *keys)
 {
   pa.old = atomicCAS(&keys[h], (K)~(K)0, key);
@@ -552,13 +559,14 @@ __device__ __forceinline__ void agg_start(PendingAdd<K, T> &pa, K key, unsigned 
   pa.on = true;
 }
 
-template <typename T, int SLOTS, typename K>
+template <typename T, int SLOTS, int SEG, typename K>
 __device__ __forceinline__ void agg_finish(PendingAdd<K, T> &pa, K *keys, T *vals, T *__restrict__ maps)
 {
   if (!pa.on) return;
   pa.on = false;
   if (pa.old == (K)~(K)0 || pa.old == pa.key) atomicAdd(&vals[pa.h], pa.val);
-  else agg_add<T, SLOTS, K>(pa.key, (pa.h + 1) & (SLOTS - 1), pa.val, keys, vals, maps, 63);
+  else agg_add<T, SLOTS, SEG, K>(pa.key, (pa.h + (1u << SEG)) & (SLOTS - 1), pa.val, keys, vals, maps,
+                                 AGG_PROBES - 1);
 }
 
 // Samples whose FP32 decision missed a margin, queued per workgroup in LDS and resolved by the FP64
@@ -598,12 +606,14 @@ __device__ __forceinline__ int resolve_deferred(const MapParams &m, double x, do
 
 // One workgroup = one TILE_X x TILE_Y x TILE_Z block of cells (one cell per thread).  Samples are
 // summed per (channel, pixel) bin in LDS and every occupied bin is added to HBM once, so the
-// global atomics scale with the bins a tile touches instead of with its samples.  SLOTS (2048, 1024 or
+// global atomics scale with the bins a tile touches instead of with its samples.  SLOTS (1024, 2048 or
 // 4096 bins) trades occupancy against probe length and overflow; SEG groups the bins of 2^SEG adjacent
 // map words (home_slot); K is the bin key type (32-bit when n_nu npix < 2^32 - 1, which halves the key
 // table).  In TABLE mode the FP32 screen decides the samples and its FP64 fallbacks are queued per workgroup.
 // FX (deterministic scatter): every sample adds the integer round(s mass / n_sub) to the 64-bit bin of
 // m.fxmaps instead of its FP mK value to maps; k_fx_finalize applies 1/s and the channel factor.
+// The VALU bounds it: 1024^3, Nside 512, 10 samples a cell 30.3 ms (33.4 with runs of slots that start anywhere and
+// up to 64 probes), 384^3 with 64 samples 7.6 (11.0), Nside 512 there 21.7 (50).
 template <typename T, int SLOTS, int SEG, bool FX, typename K>
 __device__ __forceinline__ void pixelize_body(const cx<T> *__restrict__ F, T *__restrict__ maps, const MapParams &m)
 {
@@ -660,7 +670,7 @@ __device__ __forceinline__ void pixelize_body(const cx<T> *__restrict__ F, T *__
   auto add_v = [&](int inu, int64_t ipix, V v) {
     if (inu >= 0 && (uint64_t)ipix < (uint64_t)m.npix) {
       const K key = (K)((unsigned long long)(unsigned)inu * (unsigned)m.npix + (unsigned)ipix);
-      agg_add<V, SLOTS, K>(key, home_slot<SLOTS, SEG, K>(key), v, keys, vals, vmaps);
+      agg_add<V, SLOTS, SEG, K>(key, home_slot<SLOTS, SEG, K>(key), v, keys, vals, vmaps);
     }
   };
   if (active) {
@@ -693,8 +703,8 @@ __device__ __forceinline__ void pixelize_body(const cx<T> *__restrict__ F, T *__
             run.val += v;
           }
           else {
-            agg_finish<V, SLOTS, K>(run, keys, vals, vmaps);
-            agg_start<V, SLOTS, K>(run, key, home_slot<SLOTS, SEG, K>(key), v, keys);
+            agg_finish<V, SLOTS, SEG, K>(run, keys, vals, vmaps);
+            agg_start<V, SLOTS, SEG, K>(run, key, home_slot<SLOTS, SEG, K>(key), v, keys);
           }
         }
         const unsigned long long md = __ballot(d);
@@ -723,7 +733,7 @@ __device__ __forceinline__ void pixelize_body(const cx<T> *__restrict__ F, T *__
           }
         }
       }
-      agg_finish<V, SLOTS, K>(run, keys, vals, vmaps);
+      agg_finish<V, SLOTS, SEG, K>(run, keys, vals, vmaps);
     }
     else {
       for (int isub = 0; isub < m.n_sub; isub++) {
@@ -1455,30 +1465,29 @@ static void launch_pixelize(const cx<T> *F, T *maps, const MapParams &m, hipStre
   using K64 = unsigned long long;
   const dim3 g(gx, gy), blk(256);
   // FP32 maps with 32-bit keys and at most 2048 bins fit 7 workgroups per CU in LDS: the 7-wave kernel
-  constexpr bool W7 = sizeof(T) == 4 && !FX;
-  auto run = [&](auto slots, auto seg, bool w7) {
+  constexpr bool F32 = sizeof(T) == 4 && !FX;
+  auto run = [&](auto slots, auto seg) {
     constexpr int S = decltype(slots)::value, G = decltype(seg)::value;
-    if (k32) {
-      if constexpr (W7 && S <= 2048) {
-        if (w7) {
-          hipLaunchKernelGGL((k_pixelize_w7<T, S, G, FX, unsigned>), g, blk, 0, s, F, maps, m);
-          return;
-        }
-      }
-      hipLaunchKernelGGL((k_pixelize<T, S, G, FX, unsigned>), g, blk, 0, s, F, maps, m);
-    }
-    else {
-      hipLaunchKernelGGL((k_pixelize<T, S, G, FX, K64>), g, blk, 0, s, F, maps, m);
-    }
+    if (!k32) hipLaunchKernelGGL((k_pixelize<T, S, G, FX, K64>), g, blk, 0, s, F, maps, m);
+    else if constexpr (F32) hipLaunchKernelGGL((k_pixelize_w7<T, S, G, FX, unsigned>), g, blk, 0, s, F, maps, m);
+    else hipLaunchKernelGGL((k_pixelize<T, S, G, FX, unsigned>), g, blk, 0, s, F, maps, m);
   };
-  using I2048 = std::integral_constant<int, 2048>;
   using I1024 = std::integral_constant<int, 1024>;
+  using I2048 = std::integral_constant<int, 2048>;
   using S2 = std::integral_constant<int, 2>;
   using S3 = std::integral_constant<int, 3>;
-  if (sc.pix == 1) run(I2048{}, S3{}, true);
-  else if (sc.pix == 2) run(I2048{}, S2{}, false);
-  else if (sc.pix == 3) run(I1024{}, S2{}, true);
-  else run(I2048{}, S2{}, true);
+  // The default is 2048 slots; 4096 where a tile's samples occupy more bins than that, which costs the waves of
+  // its 39 KB (FP32) or 55 KB a workgroup: 384^3, Nside 512, 200 channels, 64 samples a cell, 2810 bins: 21.7 ms
+  // against 33.4 (FP64 32.0 / 32.3, deterministic 31.4 / 34.6); 192^3, Nside 512, 27 samples, 4650 bins: 2.8 / 4.1
+  // (2.9 / 4.0, 3.3 / 4.6); 384^3, Nside 256, 1167 bins: 8.6 / 7.6 (14.1 / 8.1, 14.5 / 8.9).  With 8-byte values
+  // 2370 bins (0.37 / 0.34) and 9950 (6.6 / 6.2), which fill the larger table too, go to the smaller one.
+  const bool many = m.tile_bins > (F32 ? 2048 : 2560) && (F32 || m.tile_bins < 8192);
+  if (sc.pix == 3) run(I1024{}, S2{});
+  else if (sc.pix == 2 || (sc.pix == 0 && many)) {
+    if (k32) hipLaunchKernelGGL((k_pixelize<T, 4096, 3, FX, unsigned>), g, blk, 0, s, F, maps, m);
+    else run(I2048{}, S3{});
+  }
+  else run(I2048{}, S3{});
 }
 
 template <typename T>

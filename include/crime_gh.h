@@ -264,7 +264,7 @@ int crime_gh_set_seed(crime_gh_t *h, uint32_t seed);
  * [0, 3); 0 is the default.  FFT variants 0-2 differ in tiling with radix-16 Stockham plans; variant 3
  * is variant 0's tiling with radix-8 plans (one pass more, smaller butterflies).  All FFT variants give
  * the same fields up to the rounding of their different butterflies (variants 0-2 bit-identical).  The
- * map variants differ in the size of the LDS aggregation table (2048, 1024, 4096 bins: the atomic order
+ * map variants differ in the LDS aggregation table (1024, 2048 or 4096 bins and their grouping: the atomic order
  * of the FP32 sums changes).  Grids below N = 128 have one FFT variant (their entries read back as 0). */
 #define CRIME_GH_N_SCHED 4
 int crime_gh_get_schedule(const crime_gh_t *h, int *sched);
