@@ -258,7 +258,7 @@ __global__ __launch_bounds__((RowCfg<T, N, V>::NT)) void k_fft_x(cx<T> *__restri
 
 // ---------------------------------------------------------------------------------------------
 // P(k) estimator: forward DFT of the resident grid as conj(IDFT(conj F)) -- kx pass on conj(F),
-// then the ky and kz passes -- followed by shell binning of |delta_k|^2.
+// the ky pass, and a kz pass that bins |delta_k|^2 into shells.
 // ---------------------------------------------------------------------------------------------
 template <typename T, int N>
 __global__ __launch_bounds__((RowCfg<T, N>::NT)) void k_fft_x_conj(cx<T> *__restrict__ F,
@@ -274,48 +274,88 @@ __global__ __launch_bounds__((RowCfg<T, N>::NT)) void k_fft_x_conj(cx<T> *__rest
   Stockham<T, N, C::TC>::run(t, load, store, slot, tw);
 }
 
-template <typename T, int N>
-__global__ __launch_bounds__((ColCfg<T, N>::NT)) void k_fft_z(cx<T> *__restrict__ F, const cx<T> *__restrict__ tw)
-{
-  using C = ColCfg<T, N>;
-  __shared__ cx<T> lds[N * C::TX];
-  const int c = threadIdx.x % C::TX, t = threadIdx.x / C::TX;
-  const int kx = blockIdx.x * C::TX + c, ky = blockIdx.y;
-  const size_t n2 = (size_t)N * N;
-  cx<T> *col = F + (size_t)kx + (size_t)N * ky;
-  auto load = [&](int e) { return col[(size_t)e * n2]; };
-  auto store = [&](int e, cx<T> v) { col[(size_t)e * n2] = v; };
-  auto slot = [&](int e) -> cx<T> & { return lds[e * C::TX + c]; };
-  Stockham<T, N, C::TC>::run(t, load, store, slot, tw);
-}
-
 // G = IDFT(conj F) = conj(DFT F).  delta real => DFT(delta)_k = (DFT F_k + conj(DFT F_{-k}))/2
 // = (conj G_k + G_{-k})/2; P_est = |DFT(delta)_k|^2 L^3 / N^6 summed into |k|/dk shells of width binw.
 // acc[3*i] += P, acc[3*i+1] += |k|/dk, acc[3*i+2] += 1 (every k of the full grid).
-template <typename T>
-__global__ __launch_bounds__(256) void k_pk_bin(const cx<T> *__restrict__ G, int n, double pscale, double binw,
-                                                int nbins, double *__restrict__ acc)
+//
+// The kz pass bins where the columns stand: a workgroup transforms TX columns (kx, ky) with their mirrors
+// (-kx, -ky), so every k it holds meets its -k, and nothing is written.  Bound by HBM, 8 N^3 bytes read (FP32); with
+// a pass that wrote the columns and one that read each mode and its mirror back, 512^3 took 641 + 691 us.
+template <typename T, int N>
+struct PkCfg {
+  static constexpr int TC = ColCfg<T, N>::TC;
+  // at most 8 columns beside their mirrors and 64 KB: two workgroups or more share a CU, neighbours share lines
+  // through their XCD's L2
+  static constexpr int tx_for()
+  {
+    int tx = cmin(8, cpow2_div(N / 2));
+    while (tx > 1 && (2 * tx * N * (int)sizeof(cx<T>) > 65536 || 2 * tx * TC > 1024)) tx /= 2;
+    return tx;
+  }
+  static constexpr int TX = tx_for(), NT = 2 * TX * TC;
+  // a column's place in LDS when it is binned, padded so that the store of the columns and a wave's read along one
+  // column both spread over the banks
+  static constexpr int LZ = N + 8;
+  // kx in [0, N/2), TX of them to a tile, for every ky; then kx = N/2, TX of its ky to a tile
+  static constexpr int TILES = N / 2 / TX * N + N / TX;
+};
+
+// A workgroup takes several tiles (neighbouring workgroups of an XCD neighbouring tiles) and hands its shell sums
+// over once: a workgroup for each tile would end in 10^7 atomics on the same few hundred words.  The shells of a
+// wave's 64 places decide how many of its LDS atomics meet in one word, so a wave goes along kz.
+template <typename T, int N, int HB>
+__global__ __launch_bounds__((PkCfg<T, N>::NT)) void k_pk_z(const cx<T> *__restrict__ F, const cx<T> *__restrict__ tw,
+                                                            double pscale, double binw, int nbins,
+                                                            double *__restrict__ acc)
 {
-  __shared__ double h[3 * PK_MAX_BINS];
-  for (int i = threadIdx.x; i < 3 * nbins; i += 256) h[i] = 0;
-  __syncthreads();
-  const size_t nn = (size_t)n, n3 = nn * nn * nn;
-  const int hf = n / 2;
-  for (size_t c = (size_t)blockIdx.x * 256 + threadIdx.x; c < n3; c += (size_t)gridDim.x * 256) {
-    int kx = (int)(c % nn), ky = (int)((c / nn) % nn), kz = (int)(c / (nn * nn));
-    int ax = kx <= hf ? kx : n - kx, ay = ky <= hf ? ky : n - ky, az = kz <= hf ? kz : n - kz;
-    double kk = sqrt((double)(ax * ax + ay * ay + az * az));
-    int bin = (int)(kk / binw);
-    if (bin >= nbins) continue;
-    size_t cm = (size_t)((n - kx) % n) + nn * ((size_t)((n - ky) % n) + nn * (size_t)((n - kz) % n));
-    cx<T> g = G[c], gm = G[cm];
-    double re = 0.5 * ((double)g.x + (double)gm.x), im = 0.5 * ((double)gm.y - (double)g.y);
-    atomicAdd(&h[3 * bin], (re * re + im * im) * pscale);
-    atomicAdd(&h[3 * bin + 1], kk);
-    atomicAdd(&h[3 * bin + 2], 1.0);
+  using C = PkCfg<T, N>;
+  __shared__ cx<T> lds[C::LZ * 2 * C::TX];
+  __shared__ double h[3 * HB];
+  constexpr int NX = N / 2 / C::TX, HF = N / 2, CHUNK = (C::TILES + 7) / 8;
+  const int c = threadIdx.x % (2 * C::TX), t = threadIdx.x / (2 * C::TX);
+  const size_t n2 = (size_t)N * N;
+  for (int i = threadIdx.x; i < 3 * nbins; i += C::NT) h[i] = 0;
+  const int xcd = blockIdx.x % 8, end = cmin((xcd + 1) * CHUNK, C::TILES);
+  for (int tile = xcd * CHUNK + (int)blockIdx.x / 8; tile < end; tile += (int)gridDim.x / 8) {
+    const bool nyq = tile >= NX * N;
+    const int x0 = nyq ? HF : tile % NX * C::TX, y0 = nyq ? (tile - NX * N) * C::TX : tile / NX;
+    int kx = x0 + (nyq ? 0 : c % C::TX), ky = y0 + (nyq ? c % C::TX : 0);
+    if (c >= C::TX) {
+      kx = (N - kx) % N;
+      ky = (N - ky) % N;
+    }
+    const cx<T> *col = F + (size_t)kx + (size_t)N * ky;
+    auto load = [&](int e) { return col[(size_t)e * n2]; };
+    auto slot = [&](int e) -> cx<T> & { return lds[e * 2 * C::TX + c]; };
+    auto store = [&](int e, cx<T> v) { lds[c * C::LZ + e] = v; };   // every read through slot() has ended
+    Stockham<T, N, C::TC>::run(t, load, store, slot, tw);
+    __syncthreads();
+    for (int i = threadIdx.x; i < C::TX * (HF + 1); i += C::NT) {
+      const int q = i / (HF + 1), e = i % (HF + 1), m = (N - e) % N;
+      const int bx = x0 + (nyq ? 0 : q), by = y0 + (nyq ? q : 0), ay = by <= HF ? by : N - by;
+      const double kk = sqrt((double)(bx * bx + ay * ay + e * e));
+      const int bin = (int)(kk / binw);
+      if (bin >= nbins) continue;
+      const cx<T> *g = lds + q * C::LZ, *gm = g + C::TX * C::LZ;
+      const double re = 0.5 * ((double)g[e].x + (double)gm[m].x), im = 0.5 * ((double)gm[m].y - (double)g[e].y);
+      double p = re * re + im * im, w = 1;
+      if (e > 0 && e < HF) {   // kz = N - e beside e
+        const double re2 = 0.5 * ((double)g[m].x + (double)gm[e].x), im2 = 0.5 * ((double)gm[e].y - (double)g[m].y);
+        p += re2 * re2 + im2 * im2;
+        w = 2;
+      }
+      if (bx > 0 && !nyq) {   // the mirrors' own modes: kx = 0 and N/2 have theirs at another ky of theirs
+        p *= 2;
+        w *= 2;
+      }
+      atomicAdd(&h[3 * bin], p * pscale);
+      atomicAdd(&h[3 * bin + 1], w * kk);
+      atomicAdd(&h[3 * bin + 2], w);
+    }
+    __syncthreads();
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < 3 * nbins; i += 256)
+  for (int i = threadIdx.x; i < 3 * nbins; i += C::NT)
     if (h[i] != 0) atomicAdd(&acc[i], h[i]);
 }
 
@@ -325,12 +365,15 @@ static hipError_t launch_pk_n(cx<T> *F, const cx<T> *tw, double pscale, double b
 {
   using CC = ColCfg<T, N>;
   using RC = RowCfg<T, N>;
+  using PC = PkCfg<T, N>;
   hipLaunchKernelGGL((k_fft_x_conj<T, N>), dim3((N * N) / RC::TY), dim3(RC::NT), 0, s, F, tw);
   hipLaunchKernelGGL((k_fft_y<T, N, 0>), dim3(N / CC::TX, N), dim3(CC::NT), 0, s, F, tw, (unsigned long long *)nullptr);
-  hipLaunchKernelGGL((k_fft_z<T, N>), dim3(N / CC::TX, N), dim3(CC::NT), 0, s, F, tw);
-  size_t n3 = (size_t)N * N * N;
-  unsigned nb = (unsigned)((n3 + 255) / 256 < 8192 ? (n3 + 255) / 256 : 8192);
-  hipLaunchKernelGGL(k_pk_bin<T>, dim3(nb), dim3(256), 0, s, F, N, pscale, binw, nbins, acc);
+  // four workgroups for each CU at most, a multiple of 8 (the XCDs)
+  const unsigned nb = (unsigned)cmin((PC::TILES + 7) / 8 * 8, 1024);
+  if (nbins <= 512)
+    hipLaunchKernelGGL((k_pk_z<T, N, 512>), dim3(nb), dim3(PC::NT), 0, s, F, tw, pscale, binw, nbins, acc);
+  else
+    hipLaunchKernelGGL((k_pk_z<T, N, PK_MAX_BINS>), dim3(nb), dim3(PC::NT), 0, s, F, tw, pscale, binw, nbins, acc);
   return hipGetLastError();
 }
 
