@@ -40,7 +40,7 @@ constexpr int emax() { return sizeof(T) == 4 ? 64 : 32; }
 // 0 only for the FFT stages.
 constexpr int N_SCHED = 4;
 constexpr int N_SCHED_PIX = 4;
-constexpr int CRIME_GH_SCHED_VERSION = 7;  // bump when a variant's meaning changes (schedule cache keys)
+constexpr int CRIME_GH_SCHED_VERSION = 8;  // bump when a variant's meaning changes (schedule cache keys)
 constexpr int TUNE_MIN_N = 128;
 struct Schedule {
   int fill = 0, y = 0, x = 0, pix = 0;
@@ -72,24 +72,25 @@ struct ColCfg {
   static constexpr int NT = TX * TC;
 };
 
-// the fused fill + kz pass only writes (64-byte write requests waste nothing): a tile of at most
-// 64 KB keeps two or more workgroups per CU, so one's mode generation overlaps another's FFT; the
-// variants take other widths, and 32 KB or 128 KB tiles above 512^3.  Default against 16 columns: 256^3 FP32
-// 104 us against 128, FP64 205 against 282, 384^3 300 against 576 (with 8 threads per column)
+// the fused fill + kz pass: TX columns, half of them the mirrors of the others.  It only writes, in segments of TX / 2
+// elements whose lines its XCD's L2 puts together; a tile of at most 64 KB keeps two or more workgroups per CU, so
+// one's mode generation overlaps another's FFT.  Default and the other width, us: 8 columns up to 256^3 (256^3 FP32 55
+// against 57 with 16, FP64 114 against 123), 16 above (384^3 FP32 174 against 216 with 8, 512^3 467 against 516),
+// less where 64 KB hold fewer, but 8 up to 128 KB (1536^3 24.5 ms against 33.2 with 4 columns in 64 KB).
 template <typename T, int N, int V = 0>
 struct FillCfg {
   static constexpr int MAXR = fft_maxr(V);
   static constexpr int W = fft_tiling(V);
   static constexpr int TC = ColCfg<T, N, V>::TC;
-  // columns: columns longer than 1 KB and up to 512^3 eight of them by default (variant 0) and sixteen in variant 1, shorter and
-  // longer ones the other way round
-  static constexpr bool NARROW = 8 * TC >= 64 && N * (int)sizeof(cx<T>) > 1024 && N <= 512;
-  static constexpr int TXT = W == 2 ? 4 : ((W == 0) == NARROW ? 8 : 16);
-  static constexpr int BUDGET = W == 2 ? 131072 : (W == 0 ? 65536 : 32768);
+  // variant 1 takes the other width, variant 2 the widest that 128 KB and 1024 threads hold
+  static constexpr bool NARROW = 8 * TC >= 64 && N * (int)sizeof(cx<T>) > 1024 && N <= 256;
+  static constexpr int TXT = W == 2 ? 32 : ((W == 0) == NARROW ? 8 : 16);
+  static constexpr int BUDGET = W == 0 ? 65536 : 131072;
   static constexpr int tx_for()
   {
     int tx = cmin(TXT, cpow2_div(N));
-    while (tx > 1 && tx * ColCfg<T, N, V>::CB > BUDGET) tx /= 2;
+    while (tx > 8 && tx * ColCfg<T, N, V>::CB > BUDGET) tx /= 2;
+    while (tx > 2 && tx * ColCfg<T, N, V>::CB > 131072) tx /= 2;   // columns and their mirrors: two at least
     return tx;
   }
   static constexpr int TX = cmin(tx_for(), 1024 / TC);

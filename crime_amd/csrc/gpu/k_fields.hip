@@ -92,8 +92,6 @@ __global__ __launch_bounds__(256) void k_amp_table(FillParams f, AmpEntry<T> *__
   else tab[m] = (float)amp;
 }
 
-// F = delta + i phi_scale phi at full-grid position (kx, ky, kz), kx in [0, N) (N a compile-time
-// constant: the mirror indices are masks or constant divisions, not runtime integer divisions)
 // (A, A psi) of mode (kx, ky, kz): a function of |k|^2 only, so kz and N - kz share it
 template <typename T, int N>
 __device__ __forceinline__ cx<T> mode_amp(const FillParams &f, const AmpEntry<T> *__restrict__ amp, int kx, int ky,
@@ -116,74 +114,85 @@ __device__ __forceinline__ cx<T> mode_amp(const FillParams &f, const AmpEntry<T>
   return ab;
 }
 
-// the element from its amplitude pair ab = mode_amp(kx, ky, kz)
-template <typename T, int N>
-__device__ __forceinline__ cx<T> fill_element_a(const FillParams &f, cx<T> ab, int kx, int ky, int kz)
+// F = delta + i phi_scale phi at full-grid position (kx, ky, kz), kx in [0, N), from the amplitude pair
+// ab = mode_amp(kx, ky, kz) and the unit-variance mode g.  The products are written as fused operations of one order:
+// a mode and its mirror (g conjugate) round alike.
+template <typename T>
+__device__ __forceinline__ cx<T> fill_element(const FillParams &f, cx<T> ab, cx<T> g, int kx, int ky, int kz)
 {
-  constexpr int n = N, h = N / 2;
   if ((kx | ky | kz) == 0) return {(T)0, (T)0};
-  int myn = (n - ky) % n, mzn = (n - kz) % n;  // -k in y and z
-  cx<T> g;
-  if (kx > 0 && kx < h) {
-    g = unit_mode<T, N>(f, kx, ky, kz);
-  }
-  else if (kx > h) {
-    cx<T> m = unit_mode<T, N>(f, n - kx, myn, mzn);
-    g = {m.x, -m.y};
-  }
-  else {  // kx == 0 or kx == N/2: Hermitian part of the plane
-    cx<T> a = unit_mode<T, N>(f, kx, ky, kz), b = unit_mode<T, N>(f, kx, myn, mzn);
-    g = {(T)0.5 * (a.x + b.x), (T)0.5 * (a.y - b.y)};
-  }
   if (f.vmode == 0) {
     // delta = A g, phi_scale phi = A psi g; F = delta + i phi_scale phi = A g (1 + i psi)
-    return {ab.x * g.x - ab.y * g.y, ab.x * g.y + ab.y * g.x};
+    return {fma(ab.x, g.x, -(ab.y * g.y)), fma(ab.y, g.x, ab.x * g.y)};
   }
   // spectral velocities: with A psi = A phi_scale f0 H0 / k^2 and S_j = sin(k_j dx)/dx,
   //   grid 0: delta + i phi_scale vx = A g + i (i S_x A psi g) = (A - S_x A psi) g
   //   grid 1: phi_scale (vy + i vz)  = i S_y A psi g - S_z A psi g = A psi (-S_z + i S_y) g
   // S_j is odd in k_j, so each v_j(k) is Hermitian wherever delta_k is (the kx = 0, N/2 planes included).
   if (f.comp == 0) {
-    const T c = ab.x - (T)f.sin_dx[kx] * ab.y;
+    const T c = fma(-(T)f.sin_dx[kx], ab.y, ab.x);
     return {c * g.x, c * g.y};
   }
   const cx<T> c = {-(T)f.sin_dx[kz] * ab.y, (T)f.sin_dx[ky] * ab.y};
-  return {c.x * g.x - c.y * g.y, c.x * g.y + c.y * g.x};
+  return {fma(c.x, g.x, -(c.y * g.y)), fma(c.x, g.y, c.y * g.x)};
 }
 
 // ---------------------------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------------------------
+// A workgroup holds TX columns (kx, ky), 0 <= kx < N/2, and their mirrors (N - kx, N - ky): F there is made of the
+// conjugates of the same modes, so each mode is drawn once.  The draw (ten Philox rounds, a logarithm, a root, a
+// sine and cosine: some 300 instructions) bounds the pass.  Column kx = 0 has kx = N/2 of the same ky in its
+// mirror's place; the two are drawn after the others by all threads, two modes to an element.
 template <typename T, int N, int V>
 __global__ __launch_bounds__((FillCfg<T, N, V>::NTG)) void k_fill_z(cx<T> *__restrict__ F, FillParams f,
                                                                  const cx<T> *__restrict__ tw)
 {
   using C = FillCfg<T, N, V>;
+  constexpr int TX = C::TX / 2, NX = N / 2 / TX, h = N / 2;
   __shared__ cx<T> lds[N * C::TX];
   stamp(f.stamp, STAMP_FILL);
-  const int c = threadIdx.x % C::TX, t = threadIdx.x / C::TX;
-  // Blocks go to the XCDs round-robin (XCD = linear block index mod 8), and N / TX is a multiple of 8,
-  // so without a rotation every row's kx = 0 and kx = N/2 blocks -- whose waves run the one-draw and the
-  // two-draw (Hermitian) branches one after the other, three draws in all -- would land on XCD 0.
-  // Rotating the column block by the row spreads them over all eight.
-  const int xb = (blockIdx.x + blockIdx.y) % gridDim.x;
-  const int kx = xb * C::TX + c, ky = blockIdx.y;
+  // neighbouring tiles on one XCD: they share lines of 128 bytes, which leave its L2 whole
+  const int tile = xcd_swizzle((int)blockIdx.x, NX * N);
+  const int x0 = tile % NX * TX, ky = tile / NX, my = (N - ky) % N;
   const size_t n2 = (size_t)N * N;
-  cx<T> *col = F + (size_t)kx + (size_t)N * ky;
   // the generator is too large to unroll into the register tile: stage the modes in LDS first
   const AmpEntry<T> *amp = (const AmpEntry<T> *)f.amp;
-  // kz = e and N - e in one step: one read of their shared amplitude (a scattered gather, a cache line per
-  // lane) for two elements
-  for (int e = t; e <= N / 2; e += C::NTG / C::TX) {
-    const cx<T> ab = mode_amp<T, N>(f, amp, kx, ky, e);
-    lds[e * C::TX + c] = fill_element_a<T, N>(f, ab, kx, ky, e);
-    if (e > 0 && e < N / 2) lds[(N - e) * C::TX + c] = fill_element_a<T, N>(f, ab, kx, ky, N - e);
+  {
+    const int q = threadIdx.x % TX, kx = x0 + q;
+    // kz = e and N - e, of the column and its mirror, in one step: one read of their shared amplitude (a scattered
+    // gather, a cache line per lane) for four elements
+    for (int e = threadIdx.x / TX; e <= h; e += C::NTG / TX) {
+      if (kx == 0) continue;
+      const cx<T> ab = mode_amp<T, N>(f, amp, kx, ky, e);
+      const int m = (N - e) % N;
+      const cx<T> g = unit_mode<T, N>(f, kx, ky, e);
+      lds[e * C::TX + q] = fill_element<T>(f, ab, g, kx, ky, e);
+      lds[m * C::TX + TX + q] = fill_element<T>(f, ab, {g.x, -g.y}, N - kx, my, m);
+      if (e == 0 || e == h) continue;
+      const cx<T> g2 = unit_mode<T, N>(f, kx, ky, m);
+      lds[m * C::TX + q] = fill_element<T>(f, ab, g2, kx, ky, m);
+      lds[e * C::TX + TX + q] = fill_element<T>(f, ab, {g2.x, -g2.y}, N - kx, my, e);
+    }
+  }
+  if (x0 == 0) {
+    // kx == 0 or kx == N/2: Hermitian part of the plane
+    for (int i = threadIdx.x; i < 2 * N; i += C::NTG) {
+      const int kx = i < N ? 0 : h, kz = i % N;
+      const cx<T> ab = mode_amp<T, N>(f, amp, kx, ky, kz);
+      const cx<T> a = unit_mode<T, N>(f, kx, ky, kz), b = unit_mode<T, N>(f, kx, my, (N - kz) % N);
+      const cx<T> g = {(T)0.5 * (a.x + b.x), (T)0.5 * (a.y - b.y)};
+      lds[kz * C::TX + (i < N ? 0 : TX)] = fill_element<T>(f, ab, g, kx, ky, kz);
+    }
   }
   __syncthreads();
   if (C::NTG > C::NT && threadIdx.x >= C::NT) {   // whole waves
     Stockham<T, N, C::TC, C::MAXR>::template idle<true>();
     return;
   }
+  const int c = threadIdx.x % C::TX, t = threadIdx.x / C::TX, kx = x0 + c % TX;
+  cx<T> *col = F + (c < TX ? (size_t)kx + (size_t)N * ky
+                           : (kx == 0 ? (size_t)h + (size_t)N * ky : (size_t)(N - kx) + (size_t)N * my));
   auto load = [&](int e) { return lds[e * C::TX + c]; };
   auto store = [&](int e, cx<T> v) { col[(size_t)e * n2] = v; };
   auto slot = [&](int e) -> cx<T> & { return lds[e * C::TX + c]; };
@@ -477,7 +486,7 @@ template <typename T, int N, int V>
 static void launch_fill_v(cx<T> *F, const FillParams &f, const cx<T> *tw, hipStream_t s)
 {
   using FC = FillCfg<T, N, V>;
-  hipLaunchKernelGGL((k_fill_z<T, N, V>), dim3(N / FC::TX, N), dim3(FC::NTG), 0, s, F, f, tw);
+  hipLaunchKernelGGL((k_fill_z<T, N, V>), dim3(N / FC::TX * N), dim3(FC::NTG), 0, s, F, f, tw);
 }
 
 template <typename T, int N, int V>
