@@ -142,7 +142,8 @@ __device__ __forceinline__ cx<T> fill_element(const FillParams &f, cx<T> ab, cx<
 // ---------------------------------------------------------------------------------------------
 // A workgroup holds TX columns (kx, ky), 0 <= kx < N/2, and their mirrors (N - kx, N - ky): F there is made of the
 // conjugates of the same modes, so each mode is drawn once.  The draw (ten Philox rounds, a logarithm, a root, a
-// sine and cosine: some 300 instructions) bounds the pass.  Column kx = 0 has kx = N/2 of the same ky in its
+// sine and cosine: some 300 instructions) bounds the pass up to 512^3 (474 us, 697 with a draw for each element); above,
+// the amplitude gathers and writes a plane apart weigh as much (1024^3 5.6 ms, 6.85).  Column kx = 0 has kx = N/2 of the same ky in its
 // mirror's place; the two are drawn after the others by all threads, two modes to an element.
 template <typename T, int N, int V>
 __global__ __launch_bounds__((FillCfg<T, N, V>::NTG)) void k_fill_z(cx<T> *__restrict__ F, FillParams f,
@@ -288,8 +289,9 @@ __global__ __launch_bounds__((RowCfg<T, N>::NT)) void k_fft_x_conj(cx<T> *__rest
 // acc[3*i] += P, acc[3*i+1] += |k|/dk, acc[3*i+2] += 1 (every k of the full grid).
 //
 // The kz pass bins where the columns stand: a workgroup transforms TX columns (kx, ky) with their mirrors
-// (-kx, -ky), so every k it holds meets its -k, and nothing is written.  Bound by HBM, 8 N^3 bytes read (FP32); with
-// a pass that wrote the columns and one that read each mode and its mirror back, 512^3 took 641 + 691 us.
+// (-kx, -ky), so every k it holds meets its -k, and nothing is written.  512^3 FP32 takes 505 us for its 1.07 GB, bound
+// by the reads (segments of 64 bytes a plane apart) and the LDS sums; a pass that wrote the columns and one that read
+// each mode and its mirror back took 641 + 691, three sums for every entry instead of a quarter of them 522.
 template <typename T, int N>
 struct PkCfg {
   static constexpr int TC = ColCfg<T, N>::TC;
@@ -347,19 +349,20 @@ __global__ __launch_bounds__((PkCfg<T, N>::NT)) void k_pk_z(const cx<T> *__restr
       if (bin >= nbins) continue;
       const cx<T> *g = lds + q * C::LZ, *gm = g + C::TX * C::LZ;
       const double re = 0.5 * ((double)g[e].x + (double)gm[m].x), im = 0.5 * ((double)gm[m].y - (double)g[e].y);
-      double p = re * re + im * im, w = 1;
-      if (e > 0 && e < HF) {   // kz = N - e beside e
+      double p = re * re + im * im;
+      const bool two = e > 0 && e < HF;   // kz = N - e beside e
+      if (two) {
         const double re2 = 0.5 * ((double)g[m].x + (double)gm[e].x), im2 = 0.5 * ((double)gm[e].y - (double)g[m].y);
         p += re2 * re2 + im2 * im2;
-        w = 2;
       }
-      if (bx > 0 && !nyq) {   // the mirrors' own modes: kx = 0 and N/2 have theirs at another ky of theirs
-        p *= 2;
-        w *= 2;
+      const bool mir = bx > 0 && !nyq;    // the mirrors' own modes: kx = 0 and N/2 have theirs at another ky of theirs
+      atomicAdd(&h[3 * bin], (mir ? 2 * p : p) * pscale);
+      // the shell's count and |k| are the same for +-ky, and for ky and kz exchanged: one entry stands for all
+      if (by <= HF && e <= by) {
+        const double w = (mir ? 2.0 : 1.0) * (two ? 2.0 : 1.0) * (by > 0 && by < HF ? 2.0 : 1.0) * (e < by ? 2.0 : 1.0);
+        atomicAdd(&h[3 * bin + 1], w * kk);
+        atomicAdd(&h[3 * bin + 2], w);
       }
-      atomicAdd(&h[3 * bin], p * pscale);
-      atomicAdd(&h[3 * bin + 1], w * kk);
-      atomicAdd(&h[3 * bin + 2], w);
     }
     __syncthreads();
   }
