@@ -513,7 +513,7 @@ def main():
                     "hbm": {"bytes_per_launch": by["pixelize"], "achieved_GB/s": achieved if dom == "pixelize" else None,
                             "frac": (achieved / HBM_PEAK_GBS) if dom == "pixelize" else None},
                     "note": "VALU lane-instructions per launch from the committed SQ_INSTS_VALU profile x 64, "
-                            "divided by the live hipEvent duration; HBM bytes are the algorithmic read of the fields"}
+                            "divided by the live stage time; HBM bytes are the algorithmic read of the fields"}
         else:
             roof = {"bound": "hbm", "kernel": dom, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(args.workload).get(KERNEL_OF_STAGE[dom]),
