@@ -548,6 +548,14 @@ __global__ __launch_bounds__(256) void k_pack_weights(const float *__restrict__ 
 
 }  // namespace
 
+constexpr int PRED_SLOTS = 4, PRED_THREADS = 8;
+constexpr int PRED_MIN = 4096, PRED_DIRECT = 65536, PRED_ROWS = 65536;   // rows: see predict_impl
+
+// pinned inputs and outputs of crime_mlp_predict, and the addresses the device has them at
+struct HostRows {
+  float *x = nullptr, *y = nullptr, *x_dev = nullptr, *y_dev = nullptr;
+};
+
 struct crime_mlp {
   int max_batch = 0, device = 0;
   hipStream_t stream = nullptr;
@@ -565,11 +573,14 @@ struct crime_mlp {
   hipGraphExec_t exec = nullptr;
   int graph_batch = 0;
   int use_graph = 1;                        // 0: every step enqueued directly (crime_mlp_set_graph)
-  // crime_mlp_predict: pinned inputs and outputs of `slots` chunks of `slot_rows` rows, and the inputs' device copies
-  // (more than one slot), sent on a stream of their own
-  int slots = 0, slot_rows = 0;
-  float *hx = nullptr, *hy = nullptr, *hx_dev = nullptr, *hy_dev = nullptr, *dx = nullptr;
-  std::vector<hipEvent_t> slot_in, slot_ev;   // a slot's inputs are on the device; its outputs in hy
+  // crime_mlp_predict: pinned inputs and outputs of direct_rows rows, max_batch of them made with the handle
+  int64_t direct_rows = 0;
+  HostRows direct;
+  // and of a long call's ring of chunks, ring_rows rows in all, whose inputs a stream of its own sends to ring_dx
+  int64_t ring_rows = 0;
+  HostRows ring;
+  float *ring_dx = nullptr;
+  hipEvent_t slot_in[PRED_SLOTS] = {}, slot_ev[PRED_SLOTS] = {};   // a slot's inputs are in ring_dx; its outputs in y
   hipStream_t copy = nullptr;
   std::string err;
 };
@@ -610,17 +621,13 @@ static void drop_graph(crime_mlp *h)
   h->graph_batch = 0;
 }
 
-static void drop_slots(crime_mlp *h)
+static void drop_ring(crime_mlp *h)
 {
-  if (h->hx) (void)hipHostFree(h->hx);
-  if (h->hy) (void)hipHostFree(h->hy);
-  if (h->dx) (void)hipFree(h->dx);
-  for (hipEvent_t e : h->slot_in) (void)hipEventDestroy(e);
-  for (hipEvent_t e : h->slot_ev) (void)hipEventDestroy(e);
-  h->hx = h->hy = h->hx_dev = h->hy_dev = h->dx = nullptr;
-  h->slot_in.clear();
-  h->slot_ev.clear();
-  h->slots = h->slot_rows = 0;
+  if (h->ring.x) (void)hipHostFree(h->ring.x);
+  if (h->ring_dx) (void)hipFree(h->ring_dx);
+  h->ring = HostRows{};
+  h->ring_dx = nullptr;
+  h->ring_rows = 0;
 }
 
 extern "C" void crime_mlp_destroy(crime_mlp_t *h)
@@ -630,7 +637,12 @@ extern "C" void crime_mlp_destroy(crime_mlp_t *h)
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   if (h->copy) (void)hipStreamSynchronize(h->copy);
   drop_graph(h);
-  drop_slots(h);
+  drop_ring(h);
+  if (h->direct.x) (void)hipHostFree(h->direct.x);
+  for (int i = 0; i < PRED_SLOTS; i++) {
+    if (h->slot_in[i]) (void)hipEventDestroy(h->slot_in[i]);
+    if (h->slot_ev[i]) (void)hipEventDestroy(h->slot_ev[i]);
+  }
   if (h->copy) (void)hipStreamDestroy(h->copy);
   void *bufs[] = {h->p, h->m, h->v, h->grad, h->wf, h->wb, h->X, h->T, h->Wt, h->Y, h->hp, h->dzp,
                   h->part_in, h->part_out, h->part_b, h->st, h->loss, h->Xall, h->Tall, h->Wall};
@@ -642,28 +654,42 @@ extern "C" void crime_mlp_destroy(crime_mlp_t *h)
 
 static int nred_of(int n) { return (n + RROWS - 1) / RROWS; }
 
-constexpr int PRED_DIRECT = 4096;   // rows of a call that needs no copies (crime_mlp_predict)
-static int ensure_slots(crime_mlp *h, int slots, int rows)
+// pinned memory for `rows` rows, the outputs behind the inputs
+static int alloc_rows(crime_mlp *h, int64_t rows, HostRows *r)
 {
-  if (slots <= h->slots && rows <= h->slot_rows) return 0;
-  slots = std::max(slots, h->slots);
-  rows = std::max(rows, h->slot_rows);
-  drop_slots(h);
-  const size_t n = (size_t)slots * rows;
-  MLP_HIP(h, hipHostMalloc((void **)&h->hx, n * NIN * sizeof(float), hipHostMallocDefault));
-  MLP_HIP(h, hipHostMalloc((void **)&h->hy, n * sizeof(float), hipHostMallocDefault));
-  MLP_HIP(h, hipHostGetDevicePointer((void **)&h->hx_dev, h->hx, 0));
-  MLP_HIP(h, hipHostGetDevicePointer((void **)&h->hy_dev, h->hy, 0));
-  if (slots > 1) {
-    MLP_HIP(h, hipMalloc((void **)&h->dx, n * NIN * sizeof(float)));
-    if (!h->copy) MLP_HIP(h, hipStreamCreateWithFlags(&h->copy, hipStreamNonBlocking));
-    h->slot_in.resize(slots, nullptr);
-    h->slot_ev.resize(slots, nullptr);
-    for (hipEvent_t &e : h->slot_in) MLP_HIP(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    for (hipEvent_t &e : h->slot_ev) MLP_HIP(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  }
-  h->slots = slots;
-  h->slot_rows = rows;
+  MLP_HIP(h, hipHostMalloc((void **)&r->x, (size_t)rows * (NIN + 1) * sizeof(float), hipHostMallocDefault));
+  MLP_HIP(h, hipHostGetDevicePointer((void **)&r->x_dev, r->x, 0));
+  r->y = r->x + rows * NIN;
+  r->y_dev = r->x_dev + rows * NIN;
+  return 0;
+}
+
+static int ensure_direct(crime_mlp *h, int64_t rows)
+{
+  for (hipEvent_t &e : h->slot_ev)
+    if (!e) MLP_HIP(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  if (rows <= h->direct_rows) return 0;
+  if (h->direct.x) (void)hipHostFree(h->direct.x);
+  h->direct = HostRows{};
+  h->direct_rows = 0;
+  const int rc = alloc_rows(h, rows, &h->direct);
+  if (!rc) h->direct_rows = rows;
+  return rc;
+}
+
+static int ensure_ring(crime_mlp *h, int64_t rows)
+{
+  if (!h->copy) MLP_HIP(h, hipStreamCreateWithFlags(&h->copy, hipStreamNonBlocking));
+  for (hipEvent_t &e : h->slot_in)
+    if (!e) MLP_HIP(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  for (hipEvent_t &e : h->slot_ev)
+    if (!e) MLP_HIP(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  if (rows <= h->ring_rows) return 0;
+  drop_ring(h);
+  const int rc = alloc_rows(h, rows, &h->ring);
+  if (rc) return rc;
+  MLP_HIP(h, hipMalloc((void **)&h->ring_dx, (size_t)rows * NIN * sizeof(float)));
+  h->ring_rows = rows;
   return 0;
 }
 
@@ -702,7 +728,7 @@ static int create_impl(crime_mlp *h, int max_batch, int device)
   MLP_HIP(h, hipMemcpy(h->p, zero.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice));
   MLP_HIP(h, hipMemcpy(h->m, zero.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice));
   MLP_HIP(h, hipMemcpy(h->v, zero.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice));
-  return ensure_slots(h, 1, std::min(PRED_DIRECT, max_batch));   // a first short call finds them
+  return ensure_direct(h, std::min(PRED_DIRECT, max_batch));   // a first call finds them
 }
 
 extern "C" int crime_mlp_create(int max_batch, int device, crime_mlp_t **out)
@@ -983,26 +1009,26 @@ struct Encoders {
   }
 };
 
-// A call of up to PRED_DIRECT rows: the kernel reads the pinned inputs and writes the pinned outputs itself, no
-// copies between (256 rows: 28 us, against 42 with the two copies).  Longer ones run in chunks of PRED_ROWS: threads
-// encode (one thread would take as long as all the rest), a second stream sends a chunk's inputs while the networks
-// run on the one before, and outputs go straight to pinned memory and are handed out meanwhile.  A million rows:
-// 1.5 ms, of which 1.3 are the kernels', against 7.7 with the encoding, copies and sinh of the whole call one
-// after the other; chunks of 32768 rows with both copies on one stream 3.1, of 65536 2.5.
-constexpr int PRED_ROWS = 65536, PRED_SLOTS = 4, PRED_THREADS = 8;
-
+// Up to 2 PRED_DIRECT rows: the kernels read pinned inputs and write pinned outputs themselves, no copies between
+// (256 rows: 26 us, against 42 with two copies).  One network's rows go in four parts, of PRED_MIN rows at least, so
+// that one is encoded while the network runs on the one before: 8192 rows 47 us, 65536 171, against 64 and 236 as one
+// chunk, encoded, copied and computed in turn; 131072 rows, which go through the same memory twice, 320 against 380
+// for the ring below.  An ensemble takes them as one part, which its networks read from a device copy above PRED_MIN
+// rows (three networks, 65536 rows: 325 us; four parts 460).  The memory is the handle's from its creation unless its
+// max_batch is smaller than the call: a new handle's first 5000 rows take 58 us, and 250 with memory pinned for them.
+// Longer calls run in a ring of PRED_SLOTS chunks of PRED_ROWS rows: threads encode (one thread would take as long as
+// all the rest), a second stream sends a chunk's inputs while the networks run on the one before, and outputs go
+// straight to pinned memory and are handed out meanwhile.  A million rows: 1.35 ms, of which 1.3 are the kernels',
+// against 7.7 with the encoding, copies and sinh of the whole call one after the other.
 static int predict_impl(crime_mlp *const *hs, int nh, int64_t n, const double *x, float inv_dnu, float scale, float *y)
 {
   crime_mlp *h = hs[0];
+  // rows of one launch: an ensemble's networks leave their outputs in their handles' buffers
   int batch = PRED_ROWS;
-  for (int k = 0; k < nh; k++) batch = std::min(batch, hs[k]->max_batch);
+  if (nh > 1)
+    for (int k = 0; k < nh; k++) batch = std::min(batch, hs[k]->max_batch);
   MLP_HIP(h, hipSetDevice(h->device));
   for (int k = 1; k < nh; k++) MLP_HIP(h, hipStreamSynchronize(hs[k]->stream));  // no pending work on its buffers
-  const bool direct = n <= std::min(PRED_DIRECT, batch);
-  const int rows = direct ? (int)((n + 63) / 64 * 64) : batch;
-  const int64_t nchunks = (n + rows - 1) / rows;
-  int rc = ensure_slots(h, direct ? 1 : (int)std::max<int64_t>(2, std::min<int64_t>(PRED_SLOTS, nchunks)), rows);
-  if (rc) return rc;
   hipStream_t s = h->stream;
   // the networks on c rows of X, their spectra into Y
   auto forward = [&](int c, const float *X, float *Y) {
@@ -1016,26 +1042,54 @@ static int predict_impl(crime_mlp *const *hs, int nh, int64_t n, const double *x
     }
     hipLaunchKernelGGL(k_spectra, dim3((c + 255) / 256), dim3(256), 0, s, h->T, c, scale, Y);
   };
-  if (direct) {
-    encode_rows(x, 0, n, inv_dnu, h->hx);
-    forward((int)n, h->hx_dev, h->hy_dev);
-    MLP_HIP(h, hipGetLastError());
+  if (n <= 2 * PRED_DIRECT) {
+    const int64_t held = std::min<int64_t>(n, PRED_DIRECT);   // rows in memory at a time
+    const int rc = ensure_direct(h, (held + 63) / 64 * 64);
+    if (rc) return rc;
+    const int quarter = (int)((held + 4 * 64 - 1) / (4 * 64) * 64);
+    const int part = nh == 1 ? std::max(PRED_MIN, quarter) : batch;
+    const int64_t nparts = (n + part - 1) / part;
+    const int64_t slots = n <= held ? nparts : std::min<int64_t>(PRED_SLOTS, held / part);
+    auto count = [&](int64_t c) { return (int)std::min<int64_t>(part, n - c * part); };
+    auto hand_out = [&](int64_t c) { memcpy(y + c * part, h->direct.y + c % slots * part, count(c) * sizeof(float)); };
+    for (int64_t c = 0; c < nparts; c++) {
+      const int64_t at = c % slots * part;
+      if (c >= slots) {
+        MLP_HIP(h, hipEventSynchronize(h->slot_ev[c % slots]));
+        hand_out(c - slots);
+      }
+      const int m = count(c);
+      encode_rows(x, c * part, c * part + m, inv_dnu, h->direct.x + at * NIN);
+      const float *X = h->direct.x_dev + at * NIN;
+      if (nh > 1 && m > PRED_MIN) {
+        MLP_HIP(h, hipMemcpyAsync(h->X, h->direct.x + at * NIN, (size_t)m * NIN * sizeof(float), hipMemcpyHostToDevice, s));
+        X = h->X;
+      }
+      forward(m, X, h->direct.y_dev + at);
+      MLP_HIP(h, hipGetLastError());
+      if (c + slots < nparts) MLP_HIP(h, hipEventRecord(h->slot_ev[c % slots], s));
+    }
     MLP_HIP(h, hipStreamSynchronize(s));
-    memcpy(y, h->hy, (size_t)n * sizeof(float));
+    for (int64_t c = std::max<int64_t>(0, nparts - slots); c < nparts; c++) hand_out(c);
     return 0;
   }
-  const int slots = h->slots;
+  const int rows = batch;
+  const int64_t nchunks = (n + rows - 1) / rows;
+  const int slots = (int)std::min<int64_t>(PRED_SLOTS, nchunks);
+  int rc = ensure_ring(h, (int64_t)slots * rows);
+  if (rc) return rc;
   auto count = [&](int64_t c) { return (int)std::min<int64_t>(rows, n - c * rows); };
   auto hand_out = [&](int64_t c) -> int {
     MLP_HIP(h, hipEventSynchronize(h->slot_ev[c % slots]));
-    memcpy(y + c * rows, h->hy + (size_t)(c % slots) * rows, (size_t)count(c) * sizeof(float));
+    memcpy(y + c * rows, h->ring.y + (size_t)(c % slots) * rows, (size_t)count(c) * sizeof(float));
     return 0;
   };
-  Encoders enc(x, n, rows, slots, inv_dnu, h->hx);
-  enc.start((int)std::min<int64_t>(PRED_THREADS, n / (2 * Encoders::ENC_ROWS)));
+  Encoders enc(x, n, rows, slots, inv_dnu, h->ring.x);
+  enc.start(PRED_THREADS);
   int64_t out = 0;   // chunks handed out
   for (int64_t c = 0; c < nchunks && !rc; c++) {
-    if (c - out >= slots - 1 && c > 0) {   // the oldest slot will be needed next
+    // a slot is given back ahead of its use, for the threads, if a later chunk has use for it
+    if (c - out >= slots - 1 && out + slots < nchunks) {
       rc = hand_out(out);
       enc.give_back(out++);
       if (rc) break;
@@ -1044,11 +1098,11 @@ static int predict_impl(crime_mlp *const *hs, int nh, int64_t n, const double *x
     const size_t at = (size_t)(c % slots) * rows;
     const int m = count(c);
     // the slot's device inputs were read by a chunk that is handed out
-    MLP_HIP(h, hipMemcpyAsync(h->dx + at * NIN, h->hx + at * NIN, (size_t)m * NIN * sizeof(float), hipMemcpyHostToDevice,
-                              h->copy));
+    MLP_HIP(h, hipMemcpyAsync(h->ring_dx + at * NIN, h->ring.x + at * NIN, (size_t)m * NIN * sizeof(float),
+                              hipMemcpyHostToDevice, h->copy));
     MLP_HIP(h, hipEventRecord(h->slot_in[c % slots], h->copy));
     MLP_HIP(h, hipStreamWaitEvent(s, h->slot_in[c % slots], 0));
-    forward(m, h->dx + at * NIN, h->hy_dev + at);
+    forward(m, h->ring_dx + at * NIN, h->ring.y_dev + at);
     MLP_HIP(h, hipGetLastError());
     MLP_HIP(h, hipEventRecord(h->slot_ev[c % slots], s));
   }
