@@ -270,7 +270,7 @@ class Emulator:
             # encoding, networks and sinh in one call of the library (crime_mlp_predict)
             n = x.size // NIN
             y = np.empty(n, np.float32)
-            hs = (C.c_void_p * len(self.mlps))(*[m._h.value for m in self.mlps])
+            hs = (C.c_void_p * len(self.mlps))(*[m._h and m._h.value for m in self.mlps])   # closed: NULL
             self.mlp._check(self.mlp._lib.crime_mlp_predict(
                 hs, len(self.mlps), n, x.ctypes.data_as(_ffi._dp), np.float32(1.0 / self.dnu), np.float32(self.scale),
                 _fp(y)))
