@@ -40,7 +40,7 @@ constexpr int emax() { return sizeof(T) == 4 ? 64 : 32; }
 // 0 only for the FFT stages.
 constexpr int N_SCHED = 4;
 constexpr int N_SCHED_PIX = 4;
-constexpr int CRIME_GH_SCHED_VERSION = 8;  // bump when a variant's meaning changes (schedule cache keys)
+constexpr int CRIME_GH_SCHED_VERSION = 9;  // bump when a variant's meaning changes (schedule cache keys)
 constexpr int TUNE_MIN_N = 128;
 struct Schedule {
   int fill = 0, y = 0, x = 0, pix = 0;
@@ -50,14 +50,21 @@ struct Schedule {
 constexpr int fft_maxr(int V) { return V == 3 ? 8 : 16; }
 constexpr int fft_tiling(int V) { return V == 3 ? 0 : V; }
 
+// Threads per line of the ky and kx passes: plan_tc, or half its L/12 for FP32 lines of 3 2^7 or more elements in the
+// kx pass, and in the ky pass if a tile of 16 columns leaves its CU to others too (64 KB).  Enough waves then hide the
+// loads, and fewer threads exchange less through LDS; shorter lines, FP64 ones, and a tile alone on its CU want them all.
+template <typename T, int N>
+constexpr bool half_threads() { return sizeof(T) == 4 && N % 3 == 0 && N >= 384; }
+
 // strided (kz, ky) passes: TX adjacent columns per workgroup, TC threads per column; variants aim at
 // 16, 8 or 4 columns per tile
 template <typename T, int N, int V = 0>
 struct ColCfg {
   static constexpr int MAXR = fft_maxr(V);
   static constexpr int W = fft_tiling(V);
-  static constexpr int TC = plan_tc(N, cmax(64, N / emax<T>()), MAXR);
   static constexpr int CB = N * (int)sizeof(cx<T>);
+  // 384^3 FP32 191 us with L/24 threads a line against 199 with L/12; 768^3 1588 / 1576, 384^3 FP64 388 / 363
+  static constexpr int TC = half_threads<T, N>() && 16 * CB <= 65536 ? N / 24 : plan_tc(N, cmax(64, N / emax<T>()), MAXR);
   static constexpr int TXMAX = cmin(W == 0 ? 16 : (W == 1 ? 8 : 4), cpow2_div(N));
   static constexpr int tx_for(int budget)
   {
@@ -81,7 +88,7 @@ template <typename T, int N, int V = 0>
 struct FillCfg {
   static constexpr int MAXR = fft_maxr(V);
   static constexpr int W = fft_tiling(V);
-  static constexpr int TC = ColCfg<T, N, V>::TC;
+  static constexpr int TC = plan_tc(N, cmax(64, N / emax<T>()), MAXR);
   // variant 1 takes the other width, variant 2 the widest that 128 KB and 1024 threads hold
   static constexpr bool NARROW = 8 * TC >= 64 && N * (int)sizeof(cx<T>) > 1024 && N <= 256;
   static constexpr int TXT = W == 2 ? 32 : ((W == 0) == NARROW ? 8 : 16);
@@ -106,12 +113,14 @@ template <typename T, int N, int V = 0>
 struct RowCfg {
   static constexpr int MAXR = fft_maxr(V);
   static constexpr int W = fft_tiling(V);
-  static constexpr int TC = plan_tc(N, cmax(64, N / emax<T>()), MAXR);
+  // 768^3 FP32 1496 us with L/24 threads a row and 128 a workgroup, 1590 with L/12 and 256; 384^3 195 / 200, 1536^3
+  // 12.4 ms / 13.1; 768^3 FP64 2860 / 2736, 192^3 FP32 40.0 / 37.5
+  static constexpr int TC = half_threads<T, N>() ? N / 24 : plan_tc(N, cmax(64, N / emax<T>()), MAXR);
   static constexpr int RB = N * (int)sizeof(cx<T>);
   static constexpr int ty_for(int budget)
   {
     // grids below 128 have fewer rows than would fill 256 CUs with 256-thread workgroups
-    int ty = cmin(cmax((N < 128 ? 64 : 256) / TC, 1), cpow2_div(N * N));
+    int ty = cmin(cmax((N < 128 ? 64 : half_threads<T, N>() ? 128 : 256) / TC, 1), cpow2_div(N * N));
     while (ty > 1 && ty * RB > budget) ty /= 2;
     return ty;
   }
