@@ -1071,7 +1071,7 @@ __device__ __forceinline__ int ps_try_f32(uint32_t uhi, uint32_t whi, float maxp
 // One workgroup per map-stage tile (TILE_X x TILE_Y x TILE_Z cells, tiles in order of distance from the
 // observer).  A thread per cell draws its Poisson count; the tile's sources, numbered cell by cell, are then
 // taken PS_CHUNK at a time through three phases with a thread per source:
-//   A  position, pixel, redshift, the two SED weights without L, and the luminosity function's constants;
+//   A  position, pixel, redshift, the SED's two powers, and the luminosity function's constants;
 //   B  the luminosity by rejection: a lane whose attempt is accepted takes the next source of the chunk, so that
 //      no lane waits for the wave's longest run of attempts (one in nine is accepted);
 //   C  L in FP64, and the two terms into the workgroup's table of pixels, each occupied pixel then added to A, B
@@ -1095,7 +1095,7 @@ __global__ __launch_bounds__(256) void k_psources(const cx<T> *__restrict__ F, M
   __shared__ unsigned long long wsum[4];
   __shared__ uint32_t src_s[PS_CHUNK], pix_s[PS_CHUNK];  // source of its cell; pixel
   __shared__ uint8_t cell_s[PS_CHUNK];
-  __shared__ double fa_s[PS_CHUNK], fb_s[PS_CHUNK];      // the SED weights without L
+  __shared__ double r2z_s[PS_CHUNK], fa_s[PS_CHUNK], fb_s[PS_CHUNK];   // r^2 (1 + z) and the SED's two powers
   __shared__ union { struct { float maxpdf, c; } f; double logL; } lum_s[PS_CHUNK];
   __shared__ uint32_t next;
   const int n = m.n;
@@ -1181,10 +1181,10 @@ __global__ __launch_bounds__(256) void k_psources(const cx<T> *__restrict__ F, M
         int64_t p = screen_pixel(m, q);
         if (p == -2) p = vec2pix_ring(m.nside, px, py, pz, r);
         if ((uint64_t)p < (uint64_t)m.npix) pix = (uint32_t)p;
-        // the SED's powers of (1 + z) / 1000 from one logarithm
-        const double opz = 1.0 + zred + dz_s[lo], ly = log(opz * 1e-3), inv = 1.0 / (r * r * opz);
-        fa_s[j] = exp(-0.1 * ly) * inv;
-        fb_s[j] = 10.0 * exp(-0.75 * ly) * inv;
+        const double opz = 1.0 + zred + dz_s[lo];
+        r2z_s[j] = r * r * opz;
+        fa_s[j] = pow(opz * 1e-3, -0.1);
+        fb_s[j] = pow(opz * 1e-3, -0.75);
         // ps_lum_setup's constants in FP32
         int kz = (int)(zred * ps.inv_dz);
         kz = kz < 0 ? 0 : (kz < PS_NZ ? kz : PS_NZ - 1);
@@ -1258,8 +1258,8 @@ __global__ __launch_bounds__(256) void k_psources(const cx<T> *__restrict__ F, M
     // C
     for (int k = t; k < ns; k += 256)
       if (pix_s[k] != NOPIX) {
-        const double L = exp(lum_s[k].logL * M_LN10);
-        ps_agg_add<SLOTS>(pix_s[k], L * fa_s[k], L * fb_s[k], keys, va, vb, ps.A, ps.B);
+        const double wgt = exp(lum_s[k].logL * M_LN10) / r2z_s[k];
+        ps_agg_add<SLOTS>(pix_s[k], wgt * fa_s[k], 10.0 * wgt * fb_s[k], keys, va, vb, ps.A, ps.B);
       }
     __syncthreads();
   }
