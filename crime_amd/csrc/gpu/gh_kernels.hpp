@@ -217,8 +217,8 @@ struct MapParams {
   int nbins;
   double tile_hd;              // every cell centre of a tile lies within tile_hd of the tile's centre
   uint32_t *tile_range;        // device [first, last): the entries of tile_order the map kernel visits
-  uint8_t *tile_cull;          // device [ntiles]: 1 when tile_order's entry i is out of the band (k_map_prep;
-                               // written for the range only)
+  uint8_t *tile_cull;          // device [ntiles]: 1 when tile_order's entry i is out of the band (k_map_prep, for
+                               // every entry: its blocks run beside the one that finds the range)
   int ntx, nty, ntz;
   double tile_bins;        // estimate of the (channel, pixel) bins that a tile's samples occupy
   int vmode;               // CRIME_GH_VEL_*: SPECTRAL reads vx from F.y and (vy, vz) from G

@@ -1051,10 +1051,13 @@ __device__ __forceinline__ bool ps_try_f64(const MapParams &m, const PsParams &p
 }
 
 // Attempt `att` in FP32 from the high words of its two draws: 1 accepted, 0 rejected, -1 too close to tell.
-// u within 2^-32 + 2^-25 u, w within 2^-25; x = L / LX = 2^(q0 + q1 w) and the density c x^(alpha+1) e^-x, whose
-// exponents (at most 64 in size where x <= 64) carry 2^-19 of rounding: both sides are within 4e-6 (1 + x) of the
-// exact ones (maxpdf and c included), so a difference beyond 1e-5 (1 + x) of the larger, with 2^-30 maxpdf for
-// u, has the sign of the FP64 comparison.  Above x = 64 the density is below 1e-24 of its largest value.
+// u lies within 2^-32 + 2^-24 u of the draw, w within 2^-25 + 2^-32.  x = L / LX = 2^e, e = q0 + q1 w, carries 36.6 times
+// w's error (1.1e-6), its constants' rounding (2.2e-6) and its own (1e-6 at most): e within 3.6e-6 where x <= 64, x
+// within 2.6e-6 of itself.  The density c x^(alpha+1) e^-x has the exponent -1.45 x + 0.367 e, up to 90 in size where
+// x <= 64: 2^-18 of rounding, and 1.45 x times the error of x.  With the units of exp2, maxpdf's and c's roundings (7e-7,
+// most of it the logarithm in c) both sides together are within 2.7e-6 (1 + x) of the exact ones, so a difference beyond
+// 1e-5 (1 + x) of the larger, with 2^-30 maxpdf for u, has the sign of the FP64 comparison.  Above x = 64 the density is
+// below 1e-24 of its largest value.
 __device__ __forceinline__ int ps_try_f32(uint32_t uhi, uint32_t whi, float maxpdf, float c)
 {
   constexpr float LOG2_10 = 3.3219280948873623f, LOG2_LX = 1.0772429989324603f;
@@ -1080,7 +1083,7 @@ __device__ __forceinline__ int ps_try_f32(uint32_t uhi, uint32_t whi, float maxp
 // pixel and the luminosity function's constants are decided in FP32 with certified margins (ps_try_f32,
 // screen_pixel) and in FP64 within them: the same sources, pixels and luminosities as FP64 decisions throughout.
 // Measured: the 1024^3 box of 8300 Mpc/h (7.9e9 sources) 0.69 s against 2.85 s for a thread per cell with every
-// decision in FP64, 256^3 cells with 1.5e7 sources 2.0 ms against 14.1 ms; chunks of 256 (44 KB -> 36 KB of LDS,
+// decision in FP64, 256^3 cells with 1.5e7 sources 2.05 ms against 14.1 ms; chunks of 256 (48 KB -> 38 KB of LDS,
 // four workgroups per CU for three) 0.81 s and 2.1 ms, of 1024 (two workgroups) 0.71 s and 2.5 ms.
 constexpr int PS_CHUNK = 512;
 template <typename T>
