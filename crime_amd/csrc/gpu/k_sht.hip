@@ -745,7 +745,7 @@ __global__ __launch_bounds__(256) void k_cls_cross(const double *__restrict__ al
       }
 }
 
-// The same for 65 to 256 maps per set, one workgroup per (set, l): its 8 waves hold every 16 x 16 block of the upper
+// The same for 65 to 256 maps per set and enough l (cls_triangle_min_l), one workgroup per (set, l): its 8 waves hold every 16 x 16 block of the upper
 // triangle of C_l (NB (NB + 1) / 2 of them), so each row of alms is read once, and no block is computed twice or for
 // maps that do not exist.  8 m (16 k) pass through LDS at a time, in two buffers; the factor 2 of m > 0 is applied
 // to the sum, m = 0 entering with 1/2 (both exact).  Blocks run by falling l in groups of 16 consecutive l per XCD,
@@ -1250,11 +1250,22 @@ hipError_t launch_alm_gemm(const double *lam, const double *G, const int4 *tiles
   return hipGetLastError();
 }
 
+// Fewest l from which the triangle of nb 16 x 16 blocks to a side (5 to 16) beats the pairs of 64 x 64 tiles: one
+// workgroup to an l leaves CUs idle below 256 of them, where the tiles have 3, 6 or 10.  Stage times on both sides of the
+// lines: 80 maps, 32 l 13.3 us against 12.7, 48 l 14.2 / 15.3; 128 maps, 128 l 42.8 / 40.6, 176 l 51.3 / 53.2; 160 maps,
+// 112 l 54.4 / 47.4, 160 l 69.1 / 72.2; 192 maps, 176 l 97.7 / 87.1, 192 l 105.3 / 106.4; 256 maps, 48 l 85.1 / 30.3, 160 l
+// 149 / 133, 176 l 158 / 159, 192 l 171 / 180.
+static int cls_triangle_min_l(int nb)
+{
+  static const int16_t l[12] = {48, 80, 96, 160, 128, 144, 192, 192, 160, 176, 176, 176};
+  return l[nb - 5];
+}
+
 hipError_t launch_cls_sets(const double *alm, int lmax, int nsets, int mps, int ldo, double *cls, hipStream_t s)
 {
   const int nt = (mps + GT - 1) / GT;
   const int nl = lmax + 1;
-  if (mps > GT && mps <= 4 * GT) {
+  if (mps > GT && mps <= 4 * GT && nl >= cls_triangle_min_l((mps + 15) / 16)) {
     const int64_t nb = (int64_t)8 * nsets * (((nl + 15) / 16 + 7) / 8) * 16;
     if (nb > 0x7fffffff) return hipErrorInvalidValue;
     const dim3 g((unsigned)nb);
