@@ -539,13 +539,13 @@ static_assert(SYN_COLS == 64 || SYN_COLS == 128, "synthesis tiles of 64 or 128 c
 // it, each of its 4 waves 16 NI rows of every column with 16x16x4 FP64 MFMAs.  tile.z holds the first row and, in
 // bit 30, NI - 1: a unit's rows come in tiles of 128, the last 64 or fewer in a tile of half the height, and a wave
 // whose rows all lie beyond the unit leaves the matrix unit to the others.  C (columns in blocks of 16, at most 6)
-// is the width that covers the call's columns with the least padding (alm_col_blocks).
+// suits the call's columns and the plan's rings (alm_col_blocks).
 // A wave's Legendre rows are its own, so they go from memory to registers, 32 consecutive bytes per lane: lane
 // group g = lane / 16 holds rings 4 g .. 4 g + 3 of a 16-ring step, and the four MFMAs of the step take ring 4 g + q
 // of each group from both operands.  Only G's 16 rows pass through LDS, in two buffers with one barrier per step.
 // Rows and columns out of range are read from an in-range address and not stored: the loop has no selects.
-// What bounds it: the FP64 matrix rate, with three waves per SIMD to cover the loads.  200 maps at Nside 512: 15.6 ms, 62 TFLOP/s of the
-// 72.8 that a large library product reaches, against 18.9 ms for fixed tiles of 128 x 64 through LDS, whose padding
+// What bounds it: the FP64 matrix rate, with three waves per SIMD or more to cover the loads.  200 maps at Nside 512:
+// 15.6 ms, 62 TFLOP/s of the 72.8 that a large library product reaches, against 18.9 ms for fixed tiles of 128 x 64 through LDS, whose padding
 // (17% of the rows, 12% of the columns) was a quarter of their products.
 template <int NI, int C>
 __device__ __forceinline__ void alm_gemm_tile(const double *__restrict__ lam, const double *__restrict__ G, int m,
@@ -642,7 +642,7 @@ __device__ __forceinline__ void alm_gemm_tile(const double *__restrict__ lam, co
 }
 
 template <int C>
-__global__ __launch_bounds__(256, 3) void k_alm_gemm(const double *__restrict__ lam, const double *__restrict__ G,
+__global__ __launch_bounds__(256, C == 4 ? 4 : 3) void k_alm_gemm(const double *__restrict__ lam, const double *__restrict__ G,
                                                   const int4 *__restrict__ tiles, int ncoltiles, XcdRuns xr,
                                                   const int64_t *__restrict__ off, int m0, int lmax, int RP, int ldg,
                                                   int ncols, double *__restrict__ alm, int ldo)
@@ -1211,16 +1211,23 @@ hipError_t launch_legendre(const double2 *coef, const int64_t *off, int m0, int 
   return hipGetLastError();
 }
 
-// Column blocks (of 16) per alm GEMM tile: the width in [1, 6] that covers the columns with the fewest padded
-// blocks, each tile counted half a block more for the Legendre rows that it reads again
-static int alm_col_blocks(int ncols)
+// Column blocks (of 16) per alm GEMM tile.  One tile where five blocks hold the columns, or six and the plan has more
+// than 800 l: it reads the Legendre rows, the most of a small call's traffic, once (48 maps, lmax 1151 at Nside 384 1.90 ms,
+// 2.24 with 2 blocks; lmax 767 0.96 / 0.89).  Beyond that, at fewer than 1024 rings (RP of them): the least padding with the
+// narrowest tile, which leaves room for more waves and an even end (Nside 256: 64 maps 741 us with 2 blocks, 860 with 4; 80 maps
+// 928 / 1082 with 5; 96 maps 1061 with 3 / 1254 with 6), half a block for each tile over five, as they drift apart
+// and read the rows from memory again (128 maps 1394 with 4, 1467 with 2).  From 1024 rings on wide tiles, each counted
+// half a block more for the rows that it reads again (Nside 512: 64 maps 5.78 ms with 4 blocks, 5.95 with 2).
+static int alm_col_blocks(int ncols, int RP, int lmax)
 {
   const int nb = (ncols + 15) / 16;
+  if (nb <= (lmax < 800 ? 5 : 6)) return nb;
+  const bool narrow = RP < 1024;
   int best = 1;
   double cost = 1e300;
-  for (int c = 1; c <= 6; c++) {
+  for (int c = 2; c <= (narrow ? 5 : 6); c++) {
     const int t = (nb + c - 1) / c;
-    const double w = t * (c + 0.5);
+    const double w = narrow ? t * c + 0.5 * std::max(0, t - 5) : t * (c + 0.5);
     if (w < cost) {
       cost = w;
       best = c;
@@ -1233,7 +1240,7 @@ hipError_t launch_alm_gemm(const double *lam, const double *G, const int4 *tiles
                            const int64_t *off, int m0, int lmax, int RP, int ldg, int ncols, double *alm, int ldo,
                            hipStream_t s)
 {
-  const int c = alm_col_blocks(ncols), nct = ((ncols + 15) / 16 + c - 1) / c;
+  const int c = alm_col_blocks(ncols, RP, lmax), nct = ((ncols + 15) / 16 + c - 1) / c;
   int per_xcd = 0;
   for (int x = 0; x < 8; x++) per_xcd = std::max(per_xcd, xr.start[x + 1] - xr.start[x]);
   const dim3 g((unsigned)(8 * per_xcd * nct));
