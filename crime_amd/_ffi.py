@@ -261,6 +261,8 @@ def gpu_lib():
         lib.crime_mlp_forward_mean.argtypes = [C.POINTER(C.c_void_p), C.c_int, C.c_int64, _fp, _fp]
         lib.crime_mlp_predict.restype = C.c_int
         lib.crime_mlp_predict.argtypes = [C.POINTER(C.c_void_p), C.c_int, C.c_int64, _dp, C.c_float, C.c_float, _fp]
+        lib.crime_mlp_silu_check.restype = C.c_int
+        lib.crime_mlp_silu_check.argtypes = [H, C.POINTER(C.c_int64)]
         lib.crime_mlp_loss_grad.restype = C.c_int
         lib.crime_mlp_loss_grad.argtypes = [H, C.c_int, _fp, _fp, _fp, _dp, _fp]
         lib.crime_mlp_set_data.restype = C.c_int

@@ -67,8 +67,9 @@ __device__ __forceinline__ uint2 pack4_bf16(float a, float b, float c, float d)
   return __builtin_bit_cast(uint2, __builtin_convertvector(v, bf4));
 }
 
-// 1 / (1 + e^-z) as the correctly rounded quotient: for 1 <= d < 2^120 the reciprocal, one Newton step and two
-// residual corrections give it without the operand scaling of a general division
+// 1 / (1 + e^-z) as the correctly rounded quotient, without the operand scaling of a general division: the reciprocal
+// of 1 <= d < 2^120 by a Newton step and two residual corrections in fused arithmetic (Markstein 1990, IBM J. Res. Dev.
+// 34, 111; the quotient's bits are checked for every z by crime_mlp_silu_check)
 __device__ __forceinline__ float sigm(float z)
 {
   if (__builtin_expect(!(z > -80.0f), 0)) return 1.0f / (1.0f + expf(-z));
@@ -81,8 +82,8 @@ __device__ __forceinline__ float sigm(float z)
 
 // bf16(z sigm(z)) of four values.  Most results do not depend on the last bits of sigm: with the hardware's
 // exponential and reciprocal the product is within SILU_ULP units in the last place of z sigm(z) for z > SILU_MIN
-// (checked over every float), so unless it lies that close to a rounding boundary of BF16 its BF16 value is the
-// same.  The others (one in 2600) take sigm.
+// (its BF16 value is checked for every z by crime_mlp_silu_check), so unless it lies that close to a rounding boundary
+// of BF16 its BF16 value is the same.  The others (one in 2600) take sigm.
 constexpr unsigned SILU_ULP = 12;
 constexpr float SILU_MIN = -9.0f;
 __device__ __forceinline__ uint2 silu4_bf16(const float (&z)[4])
@@ -1200,6 +1201,41 @@ extern "C" int crime_mlp_set_data(crime_mlp_t *h, int64_t n, const float *x, con
     MLP_HIP(h, hipMemcpy(h->Wall, ones.data(), (size_t)n * sizeof(float), hipMemcpyHostToDevice));
   }
   h->ndata = n;
+  return 0;
+}
+
+// counts[0]: floats whose BF16 SiLU (a group of four of it) is not that of z sigm(z); counts[1]: whose sigm is not
+// the plain quotient; NaNs are equal to each other.  A workgroup takes 2^16 bit patterns.
+__global__ __launch_bounds__(256) void k_silu_check(unsigned long long *__restrict__ counts)
+{
+  unsigned silu = 0, quot = 0;
+  for (int i = 0; i < 256; i++) {
+    const float z = __uint_as_float(blockIdx.x * 65536u + i * 256u + threadIdx.x);
+    const float zz[4] = {z, z, z, z};
+    const uint2 a = silu4_bf16(zz);
+    const float s = sigm(z), q = 1.0f / (1.0f + expf(-z));
+    const float x = bf2f((uint16_t)a.x), y = bf2f(f2bf(z * q));
+    silu += !(x == y || (x != x && y != y)) || a.x != a.y || (a.x >> 16) != (a.x & 0xffffu);
+    quot += !(__float_as_uint(s) == __float_as_uint(q) || (s != s && q != q));
+  }
+  if (silu) atomicAdd(counts, (unsigned long long)silu);
+  if (quot) atomicAdd(counts + 1, (unsigned long long)quot);
+}
+
+extern "C" int crime_mlp_silu_check(crime_mlp_t *h, int64_t *counts)
+{
+  if (!h) return mlp_error(nullptr, CRIME_GH_EINVAL, "handle is NULL");
+  if (!counts) return mlp_error(h, CRIME_GH_EINVAL, "counts is NULL");
+  MLP_HIP(h, hipSetDevice(h->device));
+  unsigned long long zero[2] = {0, 0}, got[2], *d = (unsigned long long *)h->grad;   // scratch outside a loss_grad
+  MLP_HIP(h, hipStreamSynchronize(h->stream));
+  MLP_HIP(h, hipMemcpy(d, zero, sizeof(zero), hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(k_silu_check, dim3(65536), dim3(256), 0, h->stream, d);
+  MLP_HIP(h, hipGetLastError());
+  MLP_HIP(h, hipStreamSynchronize(h->stream));
+  MLP_HIP(h, hipMemcpy(got, d, sizeof(got), hipMemcpyDeviceToHost));
+  counts[0] = (int64_t)got[0];
+  counts[1] = (int64_t)got[1];
   return 0;
 }
 

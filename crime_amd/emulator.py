@@ -96,6 +96,12 @@ class Mlp:
         """Replay training steps as a captured graph (default) or enqueue them step by step."""
         self._check(self._lib.crime_mlp_set_graph(self._h, 1 if on else 0))
 
+    def silu_check(self):
+        """Counts of FP32 values whose BF16 SiLU, and whose sigmoid, differ from the plain formula (crime_mlp_silu_check)."""
+        c = (C.c_int64 * 2)()
+        self._check(self._lib.crime_mlp_silu_check(self._h, c))
+        return c[0], c[1]
+
     def train(self, steps, batch, lr0, total_steps, seed=0, beta1=0.9, beta2=0.999, eps=1e-8):
         loss = np.empty(steps, np.float32)
         self._check(self._lib.crime_mlp_train(self._h, steps, batch, lr0, total_steps, beta1, beta2, eps, seed,

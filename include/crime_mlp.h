@@ -13,7 +13,8 @@
  *   W0[8][256], b0[256], W1[256][256], b1[256], ..., W4[256][256], b4[256], w5[256], b5[1]
  * (W[in][out], row-major); crime_mlp_param_count() gives its length.
  *
- * A handle owns one HIP stream and its device buffers; handles are not shared across threads.
+ * A handle owns one HIP stream, its device buffers and 36 bytes of pinned host memory per row of max_batch
+ * (crime_mlp_predict); handles are not shared across threads.
  * Status codes are those of crime_gh.h.
  */
 #ifndef CRIME_MLP_H
@@ -77,6 +78,11 @@ int crime_mlp_train(crime_mlp_t *h, int steps, int batch, float lr0, int total_s
 /* on = 1 (default): crime_mlp_train replays the step as a captured HIP graph; on = 0: it enqueues the
  * same kernels step by step (the same results; for tools that trace kernel launches). */
 int crime_mlp_set_graph(crime_mlp_t *h, int on);
+
+/* Diagnostic: over every FP32 bit pattern z, counts[0] = those whose hidden-unit value, the BF16 rounding of
+ * silu(z) as the row kernel computes it from the hardware's exponential, is not that of z / (1 + expf(-z)), and
+ * counts[1] = those whose own quotient 1 / (1 + expf(-z)) is not the correctly rounded one.  Both are 0. */
+int crime_mlp_silu_check(crime_mlp_t *h, int64_t counts[2]);
 
 #ifdef __cplusplus
 }
