@@ -550,7 +550,7 @@ __global__ __launch_bounds__(256) void k_pack_weights(const float *__restrict__ 
 }  // namespace
 
 constexpr int PRED_SLOTS = 4, PRED_THREADS = 8;
-constexpr int PRED_MIN = 4096, PRED_DIRECT = 65536, PRED_ROWS = 65536;   // rows: see predict_impl
+constexpr int PRED_MIN = 4096, PRED_DIRECT = 24576, PRED_REUSE = 98304, PRED_ROWS = 65536;   // rows: see predict_impl
 
 // pinned inputs and outputs of crime_mlp_predict, and the addresses the device has them at
 struct HostRows {
@@ -1010,13 +1010,15 @@ struct Encoders {
   }
 };
 
-// Up to 2 PRED_DIRECT rows: the kernels read pinned inputs and write pinned outputs themselves, no copies between
-// (256 rows: 26 us, against 42 with two copies).  One network's rows go in four parts, of PRED_MIN rows at least, so
-// that one is encoded while the network runs on the one before: 8192 rows 47 us, 65536 171, against 64 and 236 as one
-// chunk, encoded, copied and computed in turn; 131072 rows, which go through the same memory twice, 320 against 380
-// for the ring below.  An ensemble takes them as one part, which its networks read from a device copy above PRED_MIN
-// rows (three networks, 65536 rows: 325 us; four parts 460).  The memory is the handle's from its creation unless its
-// max_batch is smaller than the call: a new handle's first 5000 rows take 58 us, and 250 with memory pinned for them.
+// Up to PRED_REUSE rows of one network: its kernels read pinned inputs and write pinned outputs themselves, no copies
+// between (256 rows: 26 us, against 42 with two copies).  The rows go in parts, so that one is encoded while the network
+// runs on the one before: quarters of the call, PRED_MIN rows at least, as long as the pinned rows hold the call, then
+// thirds of the pinned rows in turn (8192 rows, one workgroup for each CU; 6144 take as long).  8192 rows 47 us, 65536
+// 196, 98304 287, against 66, 240 and 320 as chunks that are encoded, copied and computed; 131072 370 against 350.
+// An ensemble takes up to PRED_DIRECT rows as one part, which its networks read from a device copy above PRED_MIN rows
+// (three networks, 16384 rows: 128 us; in quarters 214).  The memory is the handle's from its creation unless its
+// max_batch is smaller than the call (a new handle's first 5000 rows take 53 us, and 250 with memory pinned for
+// them), and stays below 1 MB: from there on pinning it takes 0.4 ms more.
 // Longer calls run in a ring of PRED_SLOTS chunks of PRED_ROWS rows: threads encode (one thread would take as long as
 // all the rest), a second stream sends a chunk's inputs while the networks run on the one before, and outputs go
 // straight to pinned memory and are handed out meanwhile.  A million rows: 1.35 ms, of which 1.3 are the kernels',
@@ -1043,12 +1045,12 @@ static int predict_impl(crime_mlp *const *hs, int nh, int64_t n, const double *x
     }
     hipLaunchKernelGGL(k_spectra, dim3((c + 255) / 256), dim3(256), 0, s, h->T, c, scale, Y);
   };
-  if (n <= 2 * PRED_DIRECT) {
+  if (n <= (nh == 1 ? PRED_REUSE : PRED_DIRECT)) {
     const int64_t held = std::min<int64_t>(n, PRED_DIRECT);   // rows in memory at a time
     const int rc = ensure_direct(h, (held + 63) / 64 * 64);
     if (rc) return rc;
     const int quarter = (int)((held + 4 * 64 - 1) / (4 * 64) * 64);
-    const int part = nh == 1 ? std::max(PRED_MIN, quarter) : batch;
+    const int part = nh > 1 ? batch : n > held ? PRED_DIRECT / 3 : std::max(PRED_MIN, quarter);
     const int64_t nparts = (n + part - 1) / part;
     const int64_t slots = n <= held ? nparts : std::min<int64_t>(PRED_SLOTS, held / part);
     auto count = [&](int64_t c) { return (int)std::min<int64_t>(part, n - c * part); };
@@ -1086,7 +1088,7 @@ static int predict_impl(crime_mlp *const *hs, int nh, int64_t n, const double *x
     return 0;
   };
   Encoders enc(x, n, rows, slots, inv_dnu, h->ring.x);
-  enc.start(PRED_THREADS);
+  enc.start((int)std::min<int64_t>(PRED_THREADS, n / (2 * Encoders::ENC_ROWS)));
   int64_t out = 0;   // chunks handed out
   for (int64_t c = 0; c < nchunks && !rc; c++) {
     // a slot is given back ahead of its use, for the threads, if a later chunk has use for it

@@ -13,8 +13,8 @@
  *   W0[8][256], b0[256], W1[256][256], b1[256], ..., W4[256][256], b4[256], w5[256], b5[1]
  * (W[in][out], row-major); crime_mlp_param_count() gives its length.
  *
- * A handle owns one HIP stream, its device buffers and 36 bytes of pinned host memory per row of max_batch
- * (crime_mlp_predict); handles are not shared across threads.
+ * A handle owns one HIP stream, its device buffers and pinned host memory for crime_mlp_predict (36 bytes
+ * per row of max_batch, up to 0.9 MB); handles are not shared across threads.
  * Status codes are those of crime_gh.h.
  */
 #ifndef CRIME_MLP_H

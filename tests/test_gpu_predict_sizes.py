@@ -31,11 +31,11 @@ def inputs(n):
 
 
 @pytest.mark.parametrize("nets, max_batch, sizes", [
-    (1, 65536, (16384, 16385, 65535, 65536, 65537, 131072, 131073, 300001, 5000)),
-    (1, 64, (64, 65, 4100, 20000, 131073, 70)),
-    (2, 64, (64, 65, 4100, 70000)),
-    (3, 65536, (4096, 4097, 65537)),
-    (2, 1024, (1025, 131073)),
+    (1, 65536, (16384, 16385, 24576, 24577, 65537, 98304, 98305, 300001, 5000)),
+    (1, 64, (64, 65, 4100, 24577, 98305, 70)),
+    (2, 64, (64, 65, 4100, 24577)),
+    (3, 65536, (4096, 4097, 24576, 24577, 65537)),
+    (2, 1024, (1025, 98305)),
 ])
 def test_sizes_agree(nets, max_batch, sizes):
     emu = emulator(nets, max_batch)
