@@ -224,8 +224,8 @@ class GetHI:
 
     def autotune(self, reps=3):
         """Time every variant of every stage on this handle and keep the fastest (crime_gh_autotune).
-        Returns (schedule, {stage: [ms of variant 0, 1, 2, 3]}); -1 marks a variant the grid or stage
-        lacks (variant 3, radix-8 plans, exists for the FFT stages only)."""
+        Returns (schedule, {stage: [ms of variant 0, 1, 2, 3]}); -1 marks a variant the grid lacks (the
+        FFT stages of small grids have variant 0 only)."""
         s = (C.c_int * 4)()
         nv = _ffi.N_SCHED
         ms = (C.c_double * (4 * nv))()

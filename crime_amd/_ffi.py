@@ -13,7 +13,7 @@ LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib")
 
 ABI_VERSION = 2
 NZ = 5001
-N_SCHED = 4   # CRIME_GH_N_SCHED: variants per FFT stage (the map stage has 3)
+N_SCHED = 4   # CRIME_GH_N_SCHED: variants per stage
 FP32, FP64 = 0, 1
 MODES_PHILOX, MODES_INJECTED = 0, 1
 NU_TABLE, NU_UNIFORM = 0, 1

@@ -37,7 +37,8 @@ constexpr int emax() { return sizeof(T) == 4 ? 64 : 32; }
 // (one pass more, smaller butterflies).  Map stage: LDS bins grouped by 8 adjacent map words, 2048 or 4096 as the
 // estimate of a tile's bins says (variant 0), 2048 (1) or 4096 (2; 2048 with 64-bit keys), and 1024 grouped by 4 (3).
 // Grids below TUNE_MIN_N have variant
-// 0 only for the FFT stages.
+// 0 only for the FFT stages.  Two variants can be one kernel: the map stage's variant 0 is 1 or 2, and from 768^3 FP32 up
+// the fill's variants 0 and 1 have one width.
 constexpr int N_SCHED = 4;
 constexpr int N_SCHED_PIX = 4;
 constexpr int CRIME_GH_SCHED_VERSION = 9;  // bump when a variant's meaning changes (schedule cache keys)

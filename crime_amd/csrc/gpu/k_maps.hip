@@ -612,7 +612,7 @@ __device__ __forceinline__ int resolve_deferred(const MapParams &m, double x, do
 // table).  In TABLE mode the FP32 screen decides the samples and its FP64 fallbacks are queued per workgroup.
 // FX (deterministic scatter): every sample adds the integer round(s mass / n_sub) to the 64-bit bin of
 // m.fxmaps instead of its FP mK value to maps; k_fx_finalize applies 1/s and the channel factor.
-// The VALU bounds it: 1024^3, Nside 512, 10 samples a cell 30.3 ms (33.4 with runs of slots that start anywhere and
+// The VALU bounds it: 1024^3, Nside 512, 10 samples a cell 29.1 ms (33.4 with runs of slots that start anywhere and
 // up to 64 probes), 384^3 with 64 samples 7.6 (11.0), Nside 512 there 21.7 (50).
 template <typename T, int SLOTS, int SEG, bool FX, typename K>
 __device__ __forceinline__ void pixelize_body(const cx<T> *__restrict__ F, T *__restrict__ maps, const MapParams &m)

@@ -260,8 +260,8 @@ int crime_gh_power_spectrum_noalloc(crime_gh_t *h, int nbins, double bin_dk, dou
 int crime_gh_set_seed(crime_gh_t *h, uint32_t seed);
 
 /* Kernel schedule (no counterpart in the reference): sched[4] = variants of the fill+kz pass, the ky
- * pass and the kx pass, each in [0, CRIME_GH_N_SCHED), and of the map-stage aggregation table, in
- * [0, 3); 0 is the default.  FFT variants 0-2 differ in tiling with radix-16 Stockham plans; variant 3
+ * pass and the kx pass, and of the map-stage aggregation table, each in [0, CRIME_GH_N_SCHED); 0 is the
+ * default.  FFT variants 0-2 differ in tiling with radix-16 Stockham plans; variant 3
  * is variant 0's tiling with radix-8 plans (one pass more, smaller butterflies).  All FFT variants give
  * the same fields up to the rounding of their different butterflies (variants 0-2 bit-identical).  The
  * map variants differ in the LDS aggregation table (1024, 2048 or 4096 bins and their grouping: the atomic order
